@@ -9,27 +9,28 @@
 // per stage, three stages in flight; MFMA operands (8 consecutive edges of one
 // channel per lane) come from ds_read_b64_tr_b16, which transposes 4x4 blocks
 // of 16-bit elements across each 16-lane group.
-// fp32: dw_kernel below (register transposes).
+// fp32: dw_split_kernel, on the bf16 matrix cores.  bf16 rows shorter than a
+// tile: dw_kernel (register transposes).
 //
 // With Y_e the rotated, radially scaled input rows and dZ_e the rotated output
 // gradient rows of edge e (both saved in m-major order [E, d', C] by the
 // fused kernels), the gradient of every |m| group is a GEMM with the edges as
 // the reduction axis:  C_g = sum_e dZ_g(e)^T Y_g(e), g = 0..mmax.
 //
-// Tiling.  A workgroup (4 waves) owns a 128 x 128 tile of one C_g and a
-// contiguous edge range (split-K).  Each K step covers KE edges (64 bf16 /
-// 16 fp32): every thread loads one VEC x VEC block (VEC edges x VEC columns,
-// one 16-byte load per edge, coalesced along the columns), transposes it in
-// registers and writes VEC 16-byte rows straight into MFMA fragment order, so
-// both operands are K(edge)-contiguous per lane.  Loads for step s+1 are
-// issued before the MFMAs of step s and land in the other LDS buffer (one
-// barrier per step).  Each wave computes a 64 x 64 sub-tile (2 x 2 MFMA
-// tiles of 32 x 32).  Partial tiles are summed in split order by
+// Tiling of dw_kernel.  A workgroup (4 waves) owns a 128 x 128 tile of one C_g
+// and a contiguous edge range (split-K).  Each K step covers 64 edges: every
+// thread loads one 8 x 8 block (8 edges x 8 columns, one 16-byte load per edge,
+// coalesced along the columns), transposes it in registers and writes 8 16-byte
+// rows straight into MFMA fragment order, so both operands are K(edge)-contiguous
+// per lane.  Loads for step s+1 are issued before the MFMAs of step s and land in
+// the other LDS buffer (one barrier per step).  Each wave computes a 64 x 64
+// sub-tile (2 x 2 MFMA tiles of 32 x 32).  Partial tiles are summed in split order by
 // dw_reduce_kernel, which also folds the +-m quadrants of C_m back into the
 // reference layout of so2_m_conv.fc.weight:
 //   dWr = C[+,+] + C[-,-],   dWi = C[-,+] - C[+,-]      (so2_layers.py:61-67).
 // Deterministic: no atomics.
 #include "message_impl.h"
+#include "split_bf16.h"
 #include "../../include/maloq_hip.h"
 
 namespace maloq {
@@ -61,10 +62,6 @@ struct DwCfg {
   static constexpr int NSUB = KE / KC;           // fragment columns per step
   static constexpr int FRAGS = (DW_T / 32) * NSUB;  // fragments per operand per step
   static constexpr int STAGE = 2 * FRAGS * FRAG;    // A + B bytes per step
-  // fp32: four waves per SIMD (the accumulators then live in VGPRs, 118 in
-  // all, no spills); bf16 keeps its registers (it runs only where the
-  // transpose-read kernel cannot)
-  static constexpr int MIN_WAVES = TM::VEC == 4 ? 4 : 1;
 };
 
 // Transposes a VEC x VEC block held as VEC rows of 16 bytes (row = edge,
@@ -84,17 +81,8 @@ __device__ __forceinline__ void transpose_block(const uint4 (&in)[8], uint4 (&ou
     }
   }
 }
-__device__ __forceinline__ void transpose_block(const uint4 (&in)[4], uint4 (&out)[4], F32) {
-  const uint32_t* iw = reinterpret_cast<const uint32_t*>(in);
-  uint32_t* ow = reinterpret_cast<uint32_t*>(out);
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) ow[c * 4 + e] = iw[e * 4 + c];
-}
-
 template <class TM>
-__global__ __launch_bounds__(256, DwCfg<TM>::MIN_WAVES) void dw_kernel(DwArgs a) {
+__global__ __launch_bounds__(256) void dw_kernel(DwArgs a) {
   using Cfg = DwCfg<TM>;
   constexpr int VEC = Cfg::VEC, KE = Cfg::KE, NSUB = Cfg::NSUB;
   __shared__ alignas(16) char smem[2 * Cfg::STAGE];
@@ -182,7 +170,7 @@ __global__ __launch_bounds__(256, DwCfg<TM>::MIN_WAVES) void dw_kernel(DwArgs a)
     if (more) store((s + 1) & 1);
     __syncthreads();
   }
-  float* out = a.part + split * a.goff[a.ngroups] + a.goff[g];
+  float* out = a.part + static_cast<int64_t>(split) * a.goff[a.ngroups] + a.goff[g];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int k = tk * DW_T + (2 * wk + j) * 32 + (lane & 31);
@@ -192,6 +180,160 @@ __global__ __launch_bounds__(256, DwCfg<TM>::MIN_WAVES) void dw_kernel(DwArgs a)
       for (int r = 0; r < 16; ++r) {
         const int n = tn * DW_T + (2 * wn + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
         if (n < Ng && k < Kg) out[static_cast<int64_t>(n) * Kg + k] = acc[i][j][r];
+      }
+  }
+}
+
+// ----------------------------------------------------------------- fp32
+// dw_split_kernel: the products on the bf16 matrix cores (split_bf16.h).  A
+// workgroup of 2 x 4 waves owns a 256 x 256 tile of one C_g and a contiguous
+// range of edges (split-K); a wave a 128 x 64 part.  A K step is 16
+// edges: a thread loads 8 edges of two columns (8 bytes per edge, coalesced
+// along the columns), which is what a lane of an MFMA operand holds, splits
+// them into their three bf16 planes and writes each as 16 bytes in fragment
+// order: no transposition, and each element is split once per workgroup, not
+// once per wave.  The loads of step s + 1 are in flight under the MFMAs of step
+// s and are split into the other LDS buffer between them (one barrier a step).
+//
+// What bounds it: the bf16 matrix cores (six products for one), at a rate close
+// to that of the library's large bf16 product on this card (1.16 PFLOP/s).  lmax
+// 4, mmax 2, 128 channels, 36 800 edges, 15 splits (two rounds of workgroups),
+// sums and biases included: 1350 us on the fp32 units -> 862.  One round (7 splits) takes
+// 1011: its longest workgroup has nothing beside it, and its sums are longer (error
+// 1.33e-6 against 9.0e-7; the fp32 units 1.22e-6 at their 8 splits).  128-wide tiles
+// (twice the LDS reads and splitting per product) were no faster anywhere, also on
+// small graphs (420 edges, 256 -> 128 gated: 77 us against 80).
+struct SplitDw {
+  static constexpr int T = 256, WM = 2, WN = 4;
+  static constexpr int NT = 64 * WM * WN;
+  static constexpr int KE = 16;                       // edges per K step
+  static constexpr int TI = T / WM / 32, TJ = T / WN / 32;  // a wave's MFMA tiles
+  static constexpr int OP = T / 32 * 3 * FRAG;        // bytes of one operand's planes
+  static constexpr int STAGE = 2 * OP;
+  static_assert(NT == 2 * T, "one 8-edge x 2-column block per thread");
+};
+
+__global__ __launch_bounds__(SplitDw::NT) void dw_split_kernel(DwArgs a) {
+  using S = SplitDw;
+  constexpr int T = S::T, KE = S::KE, TI = S::TI, TJ = S::TJ;
+  __shared__ alignas(16) char smem[2 * S::STAGE];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  // (32-bit and through readfirstlane: the compiler divides on the vector unit,
+  // and what follows from the quotients should stay in scalar registers)
+  const unsigned ntiles = static_cast<unsigned>(a.tile0[a.ngroups]);
+  // XCD-aware order, as in dw_tr_kernel: the tiles of one split (which read
+  // the same dZ and Y rows) run on one XCD and share its L2
+  const unsigned wid = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (wid >= ntiles * a.splits) return;  // whole workgroup, before any barrier
+  const int split = __builtin_amdgcn_readfirstlane(wid / ntiles);
+  const int t = wid - split * ntiles;
+  int g = 0;
+  while (g + 1 < a.ngroups && t >= a.tile0[g + 1]) ++g;
+  const unsigned lt = t - static_cast<unsigned>(a.tile0[g]);
+  const int tn = __builtin_amdgcn_readfirstlane(lt / static_cast<unsigned>(a.ntk[g]));
+  const int tk = lt - tn * a.ntk[g];
+  const int Ng = a.rowsz[g] * a.C_out, Kg = a.rowsy[g] * a.C_in;
+  // This thread's block: operand (0 = dZ -> A, 1 = Y -> B; uniform per wave),
+  // edges 8 eh .. 8 eh + 7 of the step, columns 2 cp and 2 cp + 1 of the tile.
+  // Buffer loads: scalar row addresses, one 32-bit offset per lane, and what lies
+  // past the last edge's row reads as zero.  Columns past the group's last are
+  // other rows' (or zero): what they give is in rows or columns of the tile that
+  // are not stored.
+  const int op = __builtin_amdgcn_readfirstlane(tid / T);
+  const int eh = __builtin_amdgcn_readfirstlane((tid % T) / (T / 2)), cp = tid % (T / 2);
+  const int C = op ? a.C_in : a.C_out;
+  const int col0 = (op ? a.row0y[g] : a.row0z[g]) * C + (op ? tk : tn) * T;  // in an edge's rows
+  const int estride = (op ? a.dpy : a.dpz) * C;
+  char* dst = smem + op * S::OP + (cp >> 4) * 3 * FRAG + (eh * 32 + 2 * (cp & 15)) * 16;
+
+  const int64_t eb = static_cast<int64_t>(split) * a.e_per_split;
+  const int64_t ee = (eb + a.e_per_split) < a.E ? (eb + a.e_per_split) : a.E;
+  const int nsteps = ee > eb ? static_cast<int>((ee - eb + KE - 1) / KE) : 0;
+  const float* src = reinterpret_cast<const float*>(op ? a.y : a.dz) + (eb + 8 * eh) * static_cast<int64_t>(estride) +
+                     col0;
+
+  float r[2][8];
+  auto load = [&](int step) {
+    const int64_t left = ee - (eb + static_cast<int64_t>(step) * KE + 8 * eh);  // edges
+    const int64_t bytes = (left * estride - col0) * 4;
+    auto rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(src + static_cast<int64_t>(step) * KE * estride), 0,
+        static_cast<int>(bytes <= 0 ? 0 : (bytes < 0x7fffffff ? bytes : 0x7fffffff)), 0x00020000);
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      const auto t2 = __builtin_amdgcn_raw_buffer_load_b64(rs, 8 * cp, v * estride * 4, 0);
+      r[0][v] = __uint_as_float(t2[0]);
+      r[1][v] = __uint_as_float(t2[1]);
+    }
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      uint4 pl[3];
+      split8(r[c], pl);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4*>(dst + buf * S::STAGE + i * FRAG + c * 16) = pl[i];
+    }
+  };
+
+  f32x16 acc[TI][TJ];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+#pragma unroll
+      for (int k = 0; k < 16; ++k) acc[i][j][k] = 0.f;
+
+  const int wm = wave / S::WN, wn = wave % S::WN;
+  const char* fa = smem + wm * TI * 3 * FRAG + lane * 16;
+  const char* fb = smem + S::OP + wn * TJ * 3 * FRAG + lane * 16;
+  auto rows = [&](int buf, int i0, int i1, const bf16x8 (&b)[TJ][3]) {
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+      if (i < i0 || i >= i1) continue;
+      bf16x8 x[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) x[k] = *reinterpret_cast<const bf16x8*>(fa + buf * S::STAGE + (i * 3 + k) * FRAG);
+#pragma unroll
+      for (int k = 0; k < SPLIT_PRODUCTS; ++k)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[split_a(k)], b[j][split_b(k)], acc[i][j], 0, 0, 0);
+    }
+  };
+  if (nsteps > 0) {
+    load(0);
+    store(0);
+    if (nsteps > 1) load(1);
+  }
+  __syncthreads();
+  for (int s = 0; s < nsteps; ++s) {
+    const int buf = s & 1;
+    bf16x8 b[TJ][3];
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) b[j][k] = *reinterpret_cast<const bf16x8*>(fb + buf * S::STAGE + (j * 3 + k) * FRAG);
+    rows(buf, 0, TI / 2, b);
+    // the other buffer was last read before the barrier that began this step
+    if (s + 1 < nsteps) {
+      store(buf ^ 1);
+      if (s + 2 < nsteps) load(s + 2);
+    }
+    rows(buf, TI / 2, TI, b);
+    __syncthreads();
+  }
+  const int row = tn * T + wm * TI * 32 + 4 * (lane >> 5);
+  float* out = a.part + static_cast<int64_t>(split) * a.goff[a.ngroups] + a.goff[g];
+#pragma unroll
+  for (int j = 0; j < TJ; ++j) {
+    const int k = tk * T + (wn * TJ + j) * 32 + (lane & 31);
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        const int n = row + i * 32 + 8 * (q >> 2) + (q & 3);
+        if (n < Ng && k < Kg) out[static_cast<int64_t>(n) * Kg + k] = acc[i][j][q];
       }
   }
 }
@@ -340,7 +482,7 @@ __global__ __launch_bounds__(256, 1) void dw_tr_kernel(DwArgs a) {
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy left in flight at exit
 
-  float* out = a.part + split * a.goff[a.ngroups] + a.goff[g];
+  float* out = a.part + static_cast<int64_t>(split) * a.goff[a.ngroups] + a.goff[g];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -480,6 +622,10 @@ extern "C" int maloq_message_dw(int dtype, int lmax, int mmax, int gate, const v
     rc = dw_setup(a, lmax, mmax, gate, num_edges, c_out, c_in, splits, trdw::T, trdw::CHUNK);
     if (rc) return rc;
   }
+  if (dtype == 0) {
+    rc = dw_setup(a, lmax, mmax, gate, num_edges, c_out, c_in, splits, SplitDw::T, SplitDw::KE);
+    if (rc) return rc;
+  }
   MALOQ_REQUIRE(partials && dw0, "null pointer");
   DwOut outm{};
   MALOQ_REQUIRE(mmax == 0 || dwm, "dwm is null");
@@ -500,7 +646,7 @@ extern "C" int maloq_message_dw(int dtype, int lmax, int mmax, int gate, const v
   else if (dtype == 1)
     hipLaunchKernelGGL(dw_kernel<BF16>, dim3(static_cast<unsigned>(grid)), dim3(256), 0, s, a);
   else
-    hipLaunchKernelGGL(dw_kernel<F32>, dim3(static_cast<unsigned>(grid)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(dw_split_kernel, dim3(static_cast<unsigned>(grid)), dim3(SplitDw::NT), 0, s, a);
   rc = check_launch("dw_kernel");
   if (rc) return rc;
   int64_t maxel = 0;

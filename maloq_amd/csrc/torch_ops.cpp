@@ -535,33 +535,19 @@ at::Tensor pack_weights(int code, int64_t lmax, int64_t mmax, bool gate, int64_t
 }
 
 // Split-K count of the weight gradient over the edges (deterministic: the
-// partials are summed in split order).  bf16: 256 x 256 output tiles, one
-// workgroup per CU, the most splits that keep every workgroup in one round;
-// fp32: 128 x 128 tiles, the count that balances the workgroups over the CUs
-// (at most four per CU, the kernel's occupancy; >= 1024 edges per split).
+// partials are summed in split order): 256 x 256 output tiles, one workgroup per
+// CU, the most splits that keep every workgroup in one round (bf16), or two from
+// 1024 edges per split on (fp32: an evener load and shorter sums).
 int dw_splits(bool bf16, int64_t lmax, int64_t mmax, bool gate, int64_t c_out, int64_t c_in, int64_t E, int cus) {
   std::vector<std::pair<int64_t, int64_t>> groups{{lmax + 1, lmax + 1}};
   for (int64_t m = 1; m <= mmax; ++m) groups.emplace_back(2 * (lmax - m + 1), 2 * (lmax - m + 1));
   if (gate) groups.emplace_back(lmax, lmax + 1);
   auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   int64_t ntiles = 0;
-  const int64_t tile = bf16 ? 256 : 128;
-  for (const auto& g : groups) ntiles += cdiv(g.first * c_out, tile) * cdiv(g.second * c_in, tile);
-  if (bf16) return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({64, cus / ntiles, cdiv(E, 128)})));
-  int best = 1;
-  double best_cost = 0;
-  bool have = false;
-  for (int s = 1; s <= 16; ++s) {
-    if (ntiles * s > 4 * cus || s > std::max<int64_t>(1, E / 1024)) continue;
-    const double cost = static_cast<double>(cdiv(ntiles * s, cus)) / s;
-    // ties go to the larger split count
-    if (!have || cost < best_cost || (cost == best_cost && s > best)) {
-      best = s;
-      best_cost = cost;
-      have = true;
-    }
-  }
-  return best;
+  for (const auto& g : groups) ntiles += cdiv(g.first * c_out, 256) * cdiv(g.second * c_in, 256);
+  int64_t splits = cus / ntiles;
+  if (!bf16) splits = std::min<int64_t>(2 * cus / ntiles, std::max<int64_t>(splits, E / 1024));
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({64, splits, cdiv(E, 128)})));
 }
 
 // Weight and bias gradients of one SO(2) convolution from the saved rows:

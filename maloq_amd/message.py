@@ -530,19 +530,14 @@ def message_weight_grad(dz, y, lmax, mmax, c_out, c_in, splits=None, num_edges=N
         groups = ([(lmax + 1, lmax + 1)] + [(2 * (lmax - m + 1),) * 2 for m in range(1, mmax + 1)]
                   + ([(lmax, lmax + 1)] if gate else []))
         cus = torch.cuda.get_device_properties(dz.device).multi_processor_count
-        if dz.dtype == torch.bfloat16:
-            # 256 x 256 tiles, one workgroup per CU: the most splits that keep
-            # every workgroup in one round
-            ntiles = sum(-(-rz * c_out // 256) * -(-ry * c_in // 256) for rz, ry in groups)
-            splits = max(1, min(64, cus // ntiles, -(-E // 128)))
-        else:
-            # 128 x 128 output tiles: the split count that balances the
-            # workgroups over the compute units (the busiest CU runs
-            # ceil(tiles * splits / CUs) of them, each 1 / splits of the edges),
-            # at most four per CU (the kernel's occupancy), >= 1024 edges per split
-            ntiles = sum(-(-rz * c_out // 128) * -(-ry * c_in // 128) for rz, ry in groups)
-            cands = [s for s in range(1, 17) if ntiles * s <= 4 * cus and s <= max(1, E // 1024)] or [1]
-            splits = min(cands, key=lambda s: (-(-ntiles * s // cus) / s, -s))
+        # 256 x 256 tiles, one workgroup per CU: the most splits that keep every
+        # workgroup in one round (bf16), or two from 1024 edges per split on (fp32:
+        # an evener load and shorter sums)
+        ntiles = sum(-(-rz * c_out // 256) * -(-ry * c_in // 256) for rz, ry in groups)
+        splits = cus // ntiles
+        if dz.dtype == torch.float32:
+            splits = min(2 * cus // ntiles, max(splits, E // 1024))
+        splits = max(1, min(64, splits, -(-E // 128)))
     lib = _lib.load()
     parts = torch.empty(max(1, lib.maloq_message_dw_partials_floats(lmax, mmax, int(gate), c_out, c_in,
                                                                     splits)),
