@@ -522,6 +522,16 @@ int maloq_edge_m0_rows(int lmax, int64_t num_edges, const float* wigner_inv, con
                        const float* jd, float* rows, void* stream);
 
 /* Node mode (edge_out == NULL): x[dst_e] += emb_e / rescale for every edge, in
+/* Weight gradient of a Linear over many rows: dw[i][j] = sum_r dy[r][i] x[r][j],
+ * dy [num_rows, n] and x [num_rows, k] fp32 with row strides ld_dy and ld_x (in
+ * floats), dw [n, k].  The fp32 kernel of maloq_message_dw; split over the rows,
+ * partials (maloq_rows_dw_partials_floats floats) summed in order: deterministic.
+ * Replaces the autograd weight gradient of the Linears of RadialMLP
+ * (helm/nn/radial.py:115-142). */
+int64_t maloq_rows_dw_partials_floats(int64_t num_rows, int n, int k);
+int maloq_rows_dw(const float* dy, int64_t ld_dy, int n, const float* x, int64_t ld_x, int k, int64_t num_rows,
+                  float* partials, float* dw, void* stream);
+
  * place, x [num_nodes, d, C]; the embedding is rounded to the dtype of x (as
  * the reference casts it) and multiplied by 1 / rescale (within one rounding
  * of the reference's division); edges are visited per node in the order

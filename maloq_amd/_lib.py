@@ -11,6 +11,7 @@ import ctypes
 import os
 
 import torch  # noqa: F401  (load torch's HIP runtime before ours)
+from torch.autograd import forward_ad
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmaloq_hip.so")
@@ -69,6 +70,8 @@ SIGNATURES = {
     "maloq_message_pack": [_i32, _i32, _p, _p, _p, _i64, _p, _p],
     "maloq_message_colsum_partials_floats": [_i32, _i32, _i64],
     "maloq_message_colsum": [_i32, _p, _i32, _i32, _i32, _i32, _i64, _p, _p, _p],
+    "maloq_rows_dw_partials_floats": [_i64, _i32, _i32],
+    "maloq_rows_dw": [_p, _i64, _i32, _p, _i64, _i32, _i64, _p, _p, _p],
     "maloq_edge_m0_rows": [_i32, _i64, _p, _p, _p, _p, _p],
     "maloq_edge_degree_embed": [_i32, _i32, _i32, _p, _i64, _i32, _p, _p, _p, _i64, ctypes.c_float, _p, _p, _p],
     "maloq_edge_degree_embed_bwd": [_i32, _i32, _p, _p, _i64, _i32, _p, ctypes.c_float, _p, _p],
@@ -90,6 +93,8 @@ RESTYPES = {
 }
 
 _lib = None
+    "maloq_rows_dw_partials_floats": ctypes.c_int64,
+    "maloq_irreps_head_partials_floats": ctypes.c_int64,
 
 
 class MaloqHipError(RuntimeError):
@@ -144,3 +149,11 @@ def require_cuda(*tensors):
     for t in tensors:
         if t is not None and not t.is_cuda:
             raise ValueError("maloq_amd HIP ops need tensors on a ROCm GPU device")
+def eager(*tensors) -> bool:
+    """Plain tensors outside torch.compile, tracing modes, functorch transforms and
+    forward-mode AD: where a call may go to a kernel that only eager code can see."""
+    return (not torch.compiler.is_compiling() and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0
+            and all(t is None or type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors))
+
+

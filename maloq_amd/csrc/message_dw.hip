@@ -44,6 +44,7 @@ struct DwArgs {
   const void* y;        // [E, dpy, C_in]
   int64_t E;
   int dpz, dpy, C_out, C_in, ngroups, splits;
+  int64_t sz, sy;       // dw_split_kernel: floats from one edge's rows to the next
   // group g: dz rows [row0z, row0z + rowsz) x y rows [row0y, row0y + rowsy)
   int row0z[MAXG], rowsz[MAXG], row0y[MAXG], rowsy[MAXG];
   int gate;                  // last group: dL/dgate rows x m = 0 rows
@@ -243,25 +244,25 @@ __global__ __launch_bounds__(SplitDw::NT) void dw_split_kernel(DwArgs a) {
   const int eh = __builtin_amdgcn_readfirstlane((tid % T) / (T / 2)), cp = tid % (T / 2);
   const int C = op ? a.C_in : a.C_out;
   const int col0 = (op ? a.row0y[g] : a.row0z[g]) * C + (op ? tk : tn) * T;  // in an edge's rows
-  const int estride = (op ? a.dpy : a.dpz) * C;
+  const int64_t estride = op ? a.sy : a.sz;
+  const int width = op ? a.dpy * a.C_in : a.dpz * a.C_out;  // of an edge's rows
   char* dst = smem + op * S::OP + (cp >> 4) * 3 * FRAG + (eh * 32 + 2 * (cp & 15)) * 16;
 
   const int64_t eb = static_cast<int64_t>(split) * a.e_per_split;
   const int64_t ee = (eb + a.e_per_split) < a.E ? (eb + a.e_per_split) : a.E;
   const int nsteps = ee > eb ? static_cast<int>((ee - eb + KE - 1) / KE) : 0;
-  const float* src = reinterpret_cast<const float*>(op ? a.y : a.dz) + (eb + 8 * eh) * static_cast<int64_t>(estride) +
-                     col0;
+  const float* src = reinterpret_cast<const float*>(op ? a.y : a.dz) + (eb + 8 * eh) * estride + col0;
 
   float r[2][8];
   auto load = [&](int step) {
     const int64_t left = ee - (eb + static_cast<int64_t>(step) * KE + 8 * eh);  // edges
-    const int64_t bytes = (left * estride - col0) * 4;
+    const int64_t bytes = left <= 0 ? 0 : ((left - 1) * estride + width - col0) * 4;
     auto rs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(src + static_cast<int64_t>(step) * KE * estride), 0,
-        static_cast<int>(bytes <= 0 ? 0 : (bytes < 0x7fffffff ? bytes : 0x7fffffff)), 0x00020000);
+        static_cast<int>(bytes < 0x7fffffff ? bytes : 0x7fffffff), 0x00020000);
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
-      const auto t2 = __builtin_amdgcn_raw_buffer_load_b64(rs, 8 * cp, v * estride * 4, 0);
+      const auto t2 = __builtin_amdgcn_raw_buffer_load_b64(rs, 8 * cp, static_cast<int>(v * estride) * 4, 0);
       r[0][v] = __uint_as_float(t2[0]);
       r[1][v] = __uint_as_float(t2[1]);
     }
@@ -512,7 +513,15 @@ __global__ void dw_reduce_kernel(DwArgs a, int lmax, float* __restrict__ dw0, Dw
   auto C = [&](int64_t n, int64_t k) {
     const float* p = a.part + a.goff[g] + n * Kg + k;
     float s = 0.f;
-    for (int sp = 0; sp < a.splits; ++sp) s += p[sp * stride];
+    int sp = 0;
+    for (; sp + 8 <= a.splits; sp += 8) {  // loads ahead of the sums, which are one chain
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = p[(sp + j) * stride];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s += v[j];
+    }
+    for (; sp < a.splits; ++sp) s += p[sp * stride];
     return s;
   };
   const bool gate_group = a.gate && g == a.ngroups - 1;
@@ -582,6 +591,8 @@ static int dw_setup(DwArgs& a, int lmax, int mmax, int gate, int64_t E, int c_ou
     a.tile0[g + 1] = a.tile0[g] + ((Ng + tile - 1) / tile) * a.ntk[g];
     a.goff[g + 1] = a.goff[g] + Ng * Kg;
   }
+  a.sz = static_cast<int64_t>(a.dpz) * c_out;
+  a.sy = static_cast<int64_t>(a.dpy) * c_in;
   a.e_per_split = ((E + splits - 1) / splits + gran - 1) / gran * gran;
   return MALOQ_OK;
 }
@@ -656,5 +667,57 @@ extern "C" int maloq_message_dw(int dtype, int lmax, int mmax, int gate, const v
   }
   hipLaunchKernelGGL(dw_reduce_kernel, dim3(static_cast<unsigned>((maxel + 255) / 256), a.ngroups),
                      dim3(256), 0, s, a, lmax, dw0, outm);
+  return check_launch("dw_reduce_kernel");
+}
+
+// ------------------------------------------------------------ plain linears
+// The weight gradient of y = x W^T over many rows, as one group of the kernel
+// above.  Splits of at least 128 rows: one workgroup per CU, two where the result
+// is a single tile (its parts are then few: 640 x 128 over 40 000 rows 94 us with
+// one, 111 with two).  What bounds it: reading dy and x once, 125 MB there, and the
+// parts, 28 MB written and read.  The library's product, a few dozen workgroups
+// over all rows, takes 243 us there, and 109 for 128 x 128 (here 46).
+static int rows_dw_splits(int64_t rows, int n, int k) {
+  const int64_t tiles = static_cast<int64_t>((n + SplitDw::T - 1) / SplitDw::T) * ((k + SplitDw::T - 1) / SplitDw::T);
+  int64_t s = (tiles > 1 ? 1 : 2) * device_cus() / tiles, most = (rows + 127) / 128;
+  s = s < most ? s : most;
+  return static_cast<int>(s < 1 ? 1 : (s < 256 ? s : 256));
+}
+
+extern "C" int64_t maloq_rows_dw_partials_floats(int64_t num_rows, int n, int k) {
+  if (num_rows < 0 || n <= 0 || k <= 0) return -1;
+  return static_cast<int64_t>(rows_dw_splits(num_rows, n, k)) * n * k;
+}
+
+extern "C" int maloq_rows_dw(const float* dy, int64_t ld_dy, int n, const float* x, int64_t ld_x, int k,
+                             int64_t num_rows, float* partials, float* dw, void* stream) {
+  MALOQ_REQUIRE(num_rows >= 0 && n > 0 && k > 0, "bad sizes");
+  MALOQ_REQUIRE(ld_dy >= n && ld_x >= k && ld_dy < (int64_t(1) << 24) && ld_x < (int64_t(1) << 24),
+                "bad row strides");
+  MALOQ_REQUIRE(partials && dw && (num_rows == 0 || (dy && x)), "null pointer");
+  DwArgs a{};
+  a.dz = dy;
+  a.y = x;
+  a.E = num_rows;
+  a.dpz = a.dpy = a.ngroups = 1;
+  a.C_out = n;
+  a.C_in = k;
+  a.splits = rows_dw_splits(num_rows, n, k);
+  a.sz = ld_dy;
+  a.sy = ld_x;
+  a.rowsz[0] = a.rowsy[0] = 1;
+  a.ntk[0] = (k + SplitDw::T - 1) / SplitDw::T;
+  a.tile0[1] = static_cast<int64_t>((n + SplitDw::T - 1) / SplitDw::T) * a.ntk[0];
+  a.goff[1] = static_cast<int64_t>(n) * k;
+  a.e_per_split = ((num_rows + a.splits - 1) / a.splits + SplitDw::KE - 1) / SplitDw::KE * SplitDw::KE;
+  a.part = partials;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int64_t grid = (a.tile0[1] * a.splits + 7) / 8 * 8;
+  MALOQ_REQUIRE(grid < (int64_t(1) << 31), "grid too large");
+  hipLaunchKernelGGL(dw_split_kernel, dim3(static_cast<unsigned>(grid)), dim3(SplitDw::NT), 0, s, a);
+  int rc = check_launch("dw_split_kernel");
+  if (rc) return rc;
+  hipLaunchKernelGGL(dw_reduce_kernel, dim3(static_cast<unsigned>((a.goff[1] + 255) / 256), 1), dim3(256), 0, s, a, 0,
+                     dw, DwOut{});
   return check_launch("dw_reduce_kernel");
 }

@@ -24,6 +24,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from . import _lib
+from .linear import linear
 
 DTYPE_CODE = {torch.float32: 0, torch.bfloat16: 1}
 
@@ -108,14 +109,14 @@ def radial_mlp(inputs: torch.Tensor, mod: RadialMLP, out_dtype: torch.dtype | No
         raise ValueError(f"inputs must be [E, {widths[0]}]")
     while len(widths) >= 3 and not fused_supported(widths):
         w1, b1, g1, bt1 = params[:4]
-        inputs = F.silu(F.layer_norm(F.linear(inputs.float(), w1, b1), (widths[1],), g1, bt1, eps))
+        inputs = F.silu(F.layer_norm(linear(inputs.float(), w1, b1), (widths[1],), g1, bt1, eps))
         widths, params = widths[1:], params[4:]
     if len(widths) < 3:    # no hidden layer left: the output Linear alone
         if dt == torch.bfloat16:
             # in the message dtype with fp32 accumulation, as the fused kernels
             # run their output layer (hidden layers stay fp32)
             return F.linear(inputs.to(dt), params[0].to(dt), params[1].to(dt))
-        return F.linear(inputs, params[0], params[1]).to(dt)
+        return linear(inputs, params[0], params[1]).to(dt)
     return _RadialFn.apply(inputs, dt, widths, eps, *params)
 
 
