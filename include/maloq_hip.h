@@ -303,6 +303,12 @@ int maloq_message_pack(int dtype, int nsrc, const float* const* srcs, const int6
 
 /* Kept rows d' = (lmax+1) + sum_{m=1..mmax} 2 (lmax-m+1) of the m-major layout,
  * and floats per edge of the kept Wigner-D rows (|m| <= mmax) in the kernels'
+/* Up to four int64 device arrays (host arrays of their pointers and sizes) to
+ * int32, truncated: array k starts at out[sum_{i < k} round_up(sizes[i], 4)].  The index
+ * arguments of the transforms above, as callers hold them, in one launch. */
+int maloq_narrow_indices(int num_arrays, const int64_t* const* arrays, const int64_t* sizes, int32_t* out,
+                         void* stream);
+
  * pair-major layout: per degree l, (l+1) column pairs (j, j+1) of the
  * nq = 1 + 2 min(mmax, l) row types, [q][2] padded to a multiple of 4 floats. */
 int maloq_message_kept_rows(int lmax, int mmax);

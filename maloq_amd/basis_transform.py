@@ -21,6 +21,8 @@ restricted to its non-zero blocks.
 """
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
 
@@ -32,6 +34,20 @@ def _i32(a, device):
     if torch.is_tensor(a):
         return a.to(device=device, dtype=torch.int32).contiguous()
     return torch.as_tensor(np.ascontiguousarray(np.asarray(a, dtype=np.int32)), device=device)
+
+
+def _i32_all(arrs, device):
+    """The arrays as int32 on ``device``; device int64 vectors in one launch."""
+    device = torch.device(device)
+    if not _lib.eager(*arrs) or not all(a.is_cuda and a.device == device and a.dtype == torch.int64
+                                        and a.dim() == 1 and a.is_contiguous() for a in arrs):
+        return tuple(_i32(a, device) for a in arrs)
+    starts = np.concatenate([[0], np.cumsum([-(-a.numel() // 4) * 4 for a in arrs])]).tolist()
+    out = torch.empty(starts[-1], device=device, dtype=torch.int32)
+    n = len(arrs)
+    _lib.call("maloq_narrow_indices", n, (ctypes.c_void_p * n)(*[a.data_ptr() for a in arrs]),
+              (ctypes.c_int64 * n)(*[a.numel() for a in arrs]), out, _lib.stream_of(device))
+    return tuple(out[s:s + a.numel()] for s, a in zip(starts, arrs))
 
 
 def _on_host(*arrs):
@@ -533,7 +549,7 @@ class HipE3TensorDecomp:
         _check_pairs_on_host(fock_block_offsets, atomic_numbers, rows, cols, fock, block_data_offsets)
         dev = fock.device
         tabs = self._template_tables(orbital_template)
-        off, Z, r_, c_ = (_i32(x, dev) for x in (fock_block_offsets, atomic_numbers, rows, cols))
+        off, Z, r_, c_ = _i32_all((fock_block_offsets, atomic_numbers, rows, cols), dev)
         ld, bdo = self._storage(fock, block_data_offsets)
         R = int(r_.shape[0])
         meta = _ops().basis_row_meta(ld, bdo, off, Z, r_, c_, tabs["pair_kind"], tabs["maxe"])
@@ -557,7 +573,7 @@ class HipE3TensorDecomp:
             raise ValueError("Unsupported dtype for the Fock matrix; only float32 is supported.")
         _check_pairs_on_host(fock_block_offsets, atomic_numbers, rows, cols, fock, block_data_offsets)
         dev = fock.device
-        off, Z, r_, c_ = (_i32(x, dev) for x in (fock_block_offsets, atomic_numbers, rows, cols))
+        off, Z, r_, c_ = _i32_all((fock_block_offsets, atomic_numbers, rows, cols), dev)
         if r_.shape != c_.shape:
             raise ValueError("rows and cols must have the same length")
         ld, bdo = self._storage(fock, block_data_offsets)

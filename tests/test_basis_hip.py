@@ -411,3 +411,17 @@ def test_wide_sorted_fock_transforms(device):
     hs.irreps_to_fock(a, Ha, off, z, rows, cols, t.orbital_template)
     hu.irreps_to_fock(b, Hb, off, z, rows, cols, t.orbital_template)
     assert torch.equal(Ha, Hb)
+
+
+@pytest.mark.parametrize("sizes", [(0, 0, 0, 0), (1, 0, 3, 4), (5, 255, 256, 257), (100003, 40, 7, 0)])
+def test_index_arrays_to_int32(sizes, device):
+    """The four index arrays of a call in one launch: equal to the conversions one
+    by one, whatever their lengths; other kinds of arrays go one by one."""
+    from maloq_amd.basis_transform import _i32_all
+    gen = torch.Generator().manual_seed(1)
+    arrs = [torch.randint(-2 ** 31, 2 ** 31, (n,), generator=gen) for n in sizes]
+    for given in ([a.to(device) for a in arrs], [a.to(device)[::2] for a in arrs], [a.to(device).int() for a in arrs],
+                  [a.numpy() for a in arrs]):
+        for got, a in zip(_i32_all(given, device), given):
+            assert got.dtype == torch.int32 and got.is_cuda
+            assert torch.equal(got.cpu(), torch.as_tensor(a).cpu().int())
