@@ -280,6 +280,12 @@ int maloq_blocks_to_csr(const float* data, const int64_t* block_data_offsets, co
                         const int64_t* block_col_offsets, const int64_t* indptr, int64_t num_blocks,
                         float* csr_data, int64_t* csr_indices, void* stream);
 
+/* Up to four int64 device arrays (host arrays of their pointers and sizes) to
+ * int32, truncated: array k starts at out[sum_{i < k} round_up(sizes[i], 4)].  The index
+ * arguments of the transforms above, as callers hold them, in one launch. */
+int maloq_narrow_indices(int num_arrays, const int64_t* const* arrays, const int64_t* sizes, int32_t* out,
+                         void* stream);
+
 /* -------------------------------------------------- fused message block -- */
 
 /* Floats of the partial-segment buffer the message entry points need. */
@@ -303,12 +309,6 @@ int maloq_message_pack(int dtype, int nsrc, const float* const* srcs, const int6
 
 /* Kept rows d' = (lmax+1) + sum_{m=1..mmax} 2 (lmax-m+1) of the m-major layout,
  * and floats per edge of the kept Wigner-D rows (|m| <= mmax) in the kernels'
-/* Up to four int64 device arrays (host arrays of their pointers and sizes) to
- * int32, truncated: array k starts at out[sum_{i < k} round_up(sizes[i], 4)].  The index
- * arguments of the transforms above, as callers hold them, in one launch. */
-int maloq_narrow_indices(int num_arrays, const int64_t* const* arrays, const int64_t* sizes, int32_t* out,
-                         void* stream);
-
  * pair-major layout: per degree l, (l+1) column pairs (j, j+1) of the
  * nq = 1 + 2 min(mmax, l) row types, [q][2] padded to a multiple of 4 floats. */
 int maloq_message_kept_rows(int lmax, int mmax);
@@ -499,6 +499,16 @@ int maloq_message_dw(int dtype, int lmax, int mmax, int gate, const void* dz, co
                      int64_t num_edges, int c_out, int c_in, int splits, float* partials,
                      float* dw0, float* const* dwm, void* stream);
 
+/* Weight gradient of a Linear over many rows: dw[i][j] = sum_r dy[r][i] x[r][j],
+ * dy [num_rows, n] and x [num_rows, k] fp32 with row strides ld_dy and ld_x (in
+ * floats), dw [n, k].  The fp32 kernel of maloq_message_dw; split over the rows,
+ * partials (maloq_rows_dw_partials_floats floats) summed in order: deterministic.
+ * Replaces the autograd weight gradient of the Linears of RadialMLP
+ * (helm/nn/radial.py:115-142). */
+int64_t maloq_rows_dw_partials_floats(int64_t num_rows, int n, int k);
+int maloq_rows_dw(const float* dy, int64_t ld_dy, int n, const float* x, int64_t ld_x, int k, int64_t num_rows,
+                  float* partials, float* dw, void* stream);
+
 /* Bias gradient of fc_m0: out[r c + k] = sum_{e < num_edges} rows[e][row0 + r][k]
  * for r < nrows, k < c, where rows [num_edges, rows_per_edge, c] (dtype 0 =
  * fp32, 1 = bf16; c a multiple of 4 resp. 8) are the saved dL/dz rows of
@@ -528,16 +538,6 @@ int maloq_edge_m0_rows(int lmax, int64_t num_edges, const float* wigner_inv, con
                        const float* jd, float* rows, void* stream);
 
 /* Node mode (edge_out == NULL): x[dst_e] += emb_e / rescale for every edge, in
-/* Weight gradient of a Linear over many rows: dw[i][j] = sum_r dy[r][i] x[r][j],
- * dy [num_rows, n] and x [num_rows, k] fp32 with row strides ld_dy and ld_x (in
- * floats), dw [n, k].  The fp32 kernel of maloq_message_dw; split over the rows,
- * partials (maloq_rows_dw_partials_floats floats) summed in order: deterministic.
- * Replaces the autograd weight gradient of the Linears of RadialMLP
- * (helm/nn/radial.py:115-142). */
-int64_t maloq_rows_dw_partials_floats(int64_t num_rows, int n, int k);
-int maloq_rows_dw(const float* dy, int64_t ld_dy, int n, const float* x, int64_t ld_x, int k, int64_t num_rows,
-                  float* partials, float* dw, void* stream);
-
  * place, x [num_nodes, d, C]; the embedding is rounded to the dtype of x (as
  * the reference casts it) and multiplied by 1 / rescale (within one rounding
  * of the reference's division); edges are visited per node in the order

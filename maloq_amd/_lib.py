@@ -48,13 +48,13 @@ SIGNATURES = {
     "maloq_label_mask": [_p, _p, _p, _p, _p, _i32, _i64, _p, _p],
     "maloq_signed_permute": [_p, _i64, _i64, _p, _p, _p, _i64, _p],
     "maloq_blocks_to_csr": [_p, _p, _p, _p, _p, _p, _p, _i64, _p, _p, _p],
+    "maloq_narrow_indices": [_i32, _p, _p, _p, _p],
     "maloq_message_partials_floats": [_i32, _i32, _i64, _i32],
     "maloq_message_wpack_bytes": [_i32, _i32, _i32, _i32, _i32, _i32],
     "maloq_message_kept_rows": [_i32, _i32],
     "maloq_message_wigner_floats": [_i32, _i32],
     "maloq_message_fwd": [_i32, _i32, _i32, _i32, _p, _i32, _p, _p, _i64, _p, _p, _p, _p, _p, _p,
                           _i64, _i32, _p, _p, _p, _p, _p, _p, _p],
-    "maloq_narrow_indices": [_i32, _p, _p, _p, _p],
     "maloq_message_edgewise_fwd": [_i32, _i32, _i32, _p, _i32, _p, _p, _p, _i64, _p, _p, _p, _p, _i32, _p, _p,
                                    _p, _p, _i64, _i32, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p],
     "maloq_message_edgewise_bwd_dx": [_i32, _i32, _i32, _p, _i32, _p, _p, _p, _p, _i64, _p, _p, _p, _p, _p, _p,
@@ -64,6 +64,8 @@ SIGNATURES = {
     "maloq_message_edge_rows": [_i64],
     "maloq_message_dw_partials_floats": [_i32, _i32, _i32, _i32, _i32, _i32],
     "maloq_message_dw": [_i32, _i32, _i32, _i32, _p, _p, _i64, _i32, _i32, _i32, _p, _p, _p, _p],
+    "maloq_rows_dw_partials_floats": [_i64, _i32, _i32],
+    "maloq_rows_dw": [_p, _i64, _i32, _p, _i64, _i32, _i64, _p, _p, _p],
     "maloq_message_supported": [_i32, _i32],
     "maloq_message_fwd_noalloc": [_i32, _i32, _i32, _i32, _p, _i32, _p, _p, _i64, _p, _p, _p, _p, _p, _p, _i64,
                                   _i32, _p, _p],
@@ -71,8 +73,6 @@ SIGNATURES = {
     "maloq_message_pack": [_i32, _i32, _p, _p, _p, _i64, _p, _p],
     "maloq_message_colsum_partials_floats": [_i32, _i32, _i64],
     "maloq_message_colsum": [_i32, _p, _i32, _i32, _i32, _i32, _i64, _p, _p, _p],
-    "maloq_rows_dw_partials_floats": [_i64, _i32, _i32],
-    "maloq_rows_dw": [_p, _i64, _i32, _p, _i64, _i32, _i64, _p, _p, _p],
     "maloq_edge_m0_rows": [_i32, _i64, _p, _p, _p, _p, _p],
     "maloq_edge_degree_embed": [_i32, _i32, _i32, _p, _i64, _i32, _p, _p, _p, _i64, ctypes.c_float, _p, _p, _p],
     "maloq_edge_degree_embed_bwd": [_i32, _i32, _p, _p, _i64, _i32, _p, ctypes.c_float, _p, _p],
@@ -87,6 +87,7 @@ RESTYPES = {
     "maloq_message_partials_floats": ctypes.c_int64,
     "maloq_message_wpack_bytes": ctypes.c_int64,
     "maloq_message_dw_partials_floats": ctypes.c_int64,
+    "maloq_rows_dw_partials_floats": ctypes.c_int64,
     "maloq_message_edge_rows": ctypes.c_int64,
     "maloq_message_colsum_partials_floats": ctypes.c_int64,
     "maloq_radial_pack_bytes": ctypes.c_int64,
@@ -94,8 +95,6 @@ RESTYPES = {
 }
 
 _lib = None
-    "maloq_rows_dw_partials_floats": ctypes.c_int64,
-    "maloq_irreps_head_partials_floats": ctypes.c_int64,
 
 
 class MaloqHipError(RuntimeError):
@@ -146,10 +145,6 @@ def stream_of(device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
-def require_cuda(*tensors):
-    for t in tensors:
-        if t is not None and not t.is_cuda:
-            raise ValueError("maloq_amd HIP ops need tensors on a ROCm GPU device")
 def eager(*tensors) -> bool:
     """Plain tensors outside torch.compile, tracing modes, functorch transforms and
     forward-mode AD: where a call may go to a kernel that only eager code can see."""
@@ -158,3 +153,7 @@ def eager(*tensors) -> bool:
             and all(t is None or type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors))
 
 
+def require_cuda(*tensors):
+    for t in tensors:
+        if t is not None and not t.is_cuda:
+            raise ValueError("maloq_amd HIP ops need tensors on a ROCm GPU device")

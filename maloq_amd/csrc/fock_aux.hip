@@ -89,8 +89,8 @@ int grid_of(int64_t n, int64_t per, unsigned* g) {
 }
 
 // Up to four int64 index arrays to int32, one after the other in out, each from a
-// multiple of 4 entries on.  What bounds it is the launch: one in place of four
-// of four conversions.  64 molecules' pair list to labels: 49 us as four, 40 so;
+// multiple of 4 entries on.  What bounds it is the launch: one in place of
+// four conversions'.  64 molecules' pair list to labels: 49 us as four, 40 so;
 // labels to four molecules' matrices: 29.3 and 27.
 struct NarrowArgs {
   const int64_t* src[4];
