@@ -226,6 +226,29 @@ int maloq_irreps_gate_fwd(const float* x, int64_t num_rows, int lmax, int c, con
 int maloq_irreps_gate_bwd(const float* x, int64_t num_rows, int lmax, int c, const float* scalars, float cst,
                           int act, const float* grad_out, float* grad_x, float* grad_scalars, void* stream);
 
+/* The whole output head of one set of rows, x [num_rows, (lmax+1)^2, c] fp32 (Fock_Irreps_Head.process
+ * and the label permutation, helm/esen_osh.py:894-1052): s = scale x_0 ws + bs with ws
+ * [c, (1+lmax) c] (bs may be null), the gate as in maloq_irreps_gate_fwd, y_l = scale gated
+ * x_l wl[l] with wl[l] [c, mul[l]] (host arrays of lmax + 1 device pointers and counts; b0 [mul[0]] added to y_0, may be null), y_l being columns
+ * sum_{k<l} (2k+1) mul[k] + m mul[l] + v, and out[r][j] = src[j] >= 0 ? sign[j] y[r][src[j]] : 0, j < t.
+ * scalars [num_rows, (1+lmax) c]: s for the backward (may be null).  Built for lmax 2, 4, 6,
+ * c 32, 64, 96, 128, up to 32 copies of a degree and 256 columns of y
+ * (maloq_irreps_head_supported); 16-byte aligned x. */
+int maloq_irreps_head_supported(int lmax, int c, const int* mul);
+int maloq_irreps_head_fwd(const float* x, int64_t num_rows, int lmax, int c, const float* ws, const float* bs,
+                          const float* const* wl, const int* mul, const float* b0, float scale, float cst, int act,
+                          const int32_t* src, const float* sign, int t, float* scalars, float* out, void* stream);
+
+/* Its gradients: grad_x, grad_scalars (of s: that of ws is scale x_0^T grad_scalars, of
+ * bs its column sums), and grad_wl: the [c, mul[l]] gradients one after the other, then that of b0 [mul[0]].  ptr, cols, csign: CSR of
+ * the gather's transpose (as in maloq_scatter_columns).  partials: maloq_irreps_head_partials_floats
+ * floats.  Fixed-order sums: deterministic.  num_rows > 0. */
+int64_t maloq_irreps_head_partials_floats(int64_t num_rows, int lmax, int c, const int* mul);
+int maloq_irreps_head_bwd(const float* x, int64_t num_rows, int lmax, int c, const float* ws,
+                          const float* const* wl, const int* mul, float scale, float cst, int act, const float* scalars,
+                          const float* grad_out, int t, const int32_t* ptr, const int32_t* cols, const float* csign,
+                          float* partials, float* grad_x, float* grad_scalars, float* grad_wl, void* stream);
+
 /* out[r, k] = src[k] >= 0 ? sign[k] in[r, src[k]] : 0 for k < t (row strides
  * ld_in, ld_out): the head's output permutation to label order
  * (x_out[:, output_permutation], esen_osh.py:909-914, 948-953), with the parity

@@ -33,6 +33,12 @@ SIGNATURES = {
     "maloq_basis_cg_block": [_i32, _p, _i32],
     "maloq_irreps_gate_fwd": [_p, _i64, _i32, _i32, _p, ctypes.c_float, _i32, _p, _p],
     "maloq_irreps_gate_bwd": [_p, _i64, _i32, _i32, _p, ctypes.c_float, _i32, _p, _p, _p, _p],
+    "maloq_irreps_head_supported": [_i32, _i32, _p],
+    "maloq_irreps_head_fwd": [_p, _i64, _i32, _i32, _p, _p, _p, _p, _p, ctypes.c_float, ctypes.c_float, _i32, _p, _p,
+                              _i32, _p, _p, _p],
+    "maloq_irreps_head_partials_floats": [_i64, _i32, _i32, _p],
+    "maloq_irreps_head_bwd": [_p, _i64, _i32, _i32, _p, _p, _p, ctypes.c_float, ctypes.c_float, _i32, _p, _p, _i32, _p,
+                              _p, _p, _p, _p, _p, _p, _p],
     "maloq_gather_columns": [_p, _i64, _i64, _p, _p, _i32, _p, _i64, _p],
     "maloq_scatter_columns": [_p, _i64, _i64, _p, _p, _p, _i32, _p, _i64, _p],
     "maloq_basis_row_meta": [_i64, _p, _p, _p, _p, _p, _i64, _p, _i32, _p, _p],
@@ -88,6 +94,7 @@ RESTYPES = {
     "maloq_message_wpack_bytes": ctypes.c_int64,
     "maloq_message_dw_partials_floats": ctypes.c_int64,
     "maloq_rows_dw_partials_floats": ctypes.c_int64,
+    "maloq_irreps_head_partials_floats": ctypes.c_int64,
     "maloq_message_edge_rows": ctypes.c_int64,
     "maloq_message_colsum_partials_floats": ctypes.c_int64,
     "maloq_radial_pack_bytes": ctypes.c_int64,

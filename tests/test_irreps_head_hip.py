@@ -202,3 +202,59 @@ def test_reduce_edge_needs_reverse_edges():
     n, e = mod({"node_embeddings": x, "edge_embeddings": torch.zeros(0, (lmax + 1) ** 2, C).cuda()},
                {"edge_index": torch.zeros(2, 0, dtype=torch.int64).cuda()})
     assert n.shape == (1, 3, T) and e.shape == (1, 0, T)
+
+
+def _close(got, ref, tol, what):
+    err = ((got.double().cpu() - ref).norm() / ref.norm()).item()
+    assert err < tol, f"{what}: rel err {err:.2e}"
+
+
+# Few copies: every gather row; many: both tiles of 16 copies.  Row counts around
+# the 32-row tile, and enough that the persistent workgroups take several.
+@pytest.mark.parametrize("lmax,mul", [(2, [5, 3, 1]), (2, [32, 16, 17]), (4, [14, 21, 15, 5, 1]),
+                                      (4, [3, 0, 16, 1, 0]), (6, [4, 9, 8, 5, 3, 2, 1])])
+@pytest.mark.parametrize("C,rows", [(32, 1), (64, 31), (96, 33), (128, 32), (128, 300), (32, 50000)])
+def test_fused_labels_match_the_layers(lmax, mul, C, rows):
+    """The one-launch head against the formulas in 64 bits, labels and every
+    gradient, and a gradient of a gradient against the unfused layers'.  Tolerance:
+    sums of C and of rows products in fp32 (n 2^-25 sqrt(n) / n rms each), eight
+    times over, and a few roundings of the gate."""
+    from maloq_amd import irreps_head as ih
+    gen = torch.Generator().manual_seed(rows + C + lmax)
+    rand = lambda *s: torch.randn(*s, generator=gen)
+    d, W, Zw = (lmax + 1) ** 2, (lmax + 1) * C, sum((2 * l + 1) * m for l, m in enumerate(mul))
+    act = rows % 2
+    src = np.concatenate([np.random.default_rng(C).permutation(Zw), [-1, 0]])  # one column twice, one empty
+    sign = np.where(np.arange(Zw + 2) % 3, 1.0, -1.0).astype(np.float32)
+    cmap = ih._ColumnMap(src, sign, Zw, "cuda")
+    host = [rand(rows, d, C), rand(C, W), rand(W), rand(mul[0])] + [rand(C, m) if m else None for m in mul]
+    dev = [None if t is None else t.cuda().requires_grad_() for t in host]
+    ref = [None if t is None else t.double().requires_grad_() for t in host]
+    out = ih._HeadFn.apply(*dev[:4], cmap, lmax, act, *dev[4:])
+
+    x, ws, bs, b0, *wls = ref
+    s = (x[:, 0] @ ws / C ** 0.5 + bs).view(rows, lmax + 1, C)
+    gate = ih._cst(act) * (torch.tanh(s.abs()) if act else torch.sigmoid(s))
+    z = []
+    for l, w in enumerate(wls):
+        if w is None:
+            continue
+        xl = s[:, :1] if l == 0 else gate[:, l:l + 1] * x[:, l * l:(l + 1) ** 2]
+        z.append((xl @ w / C ** 0.5 + (b0 if l == 0 else 0)).reshape(rows, -1))
+    z = torch.cat([torch.cat(z, 1), torch.zeros(rows, 1, dtype=torch.float64)], 1)
+    want = z[:, torch.as_tensor(src)] * torch.as_tensor(sign)
+    n = max(C, rows)
+    tol = 8 * (4 + n ** 0.5) * 2.0 ** -25
+    _close(out.detach(), want.detach(), tol, "labels")
+    g = rand(rows, len(src))
+    leaves = lambda ts: [t for t in ts if t is not None]
+    got = torch.autograd.grad(out, leaves(dev), g.cuda(), retain_graph=rows < 100)
+    for k, (a, b) in enumerate(zip(got, torch.autograd.grad(want, leaves(ref), g.double()))):
+        _close(a, b, tol, f"gradient {k}")
+    if rows < 100:
+        gw = torch.autograd.grad(out, dev[6], g.cuda(), create_graph=True)[0]
+        zu = ih._Gather.apply(ih._z_rows(dev[0], dev[1] / C ** 0.5, *dev[2:4],
+                                         [None if w is None else w / C ** 0.5 for w in dev[4:]], lmax, act), cmap)
+        gu = torch.autograd.grad(zu, dev[6], g.cuda(), create_graph=True)[0]
+        assert torch.allclose(torch.autograd.grad(gw.square().sum(), dev[0])[0],
+                              torch.autograd.grad(gu.square().sum(), dev[0])[0], rtol=1e-4, atol=1e-5 * gu.abs().max().item() ** 2)
