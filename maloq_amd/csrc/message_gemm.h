@@ -23,14 +23,23 @@
 //         y+ = Wr x+ - Wi x-,  y- = Wi x+ + Wr x-        (so2_layers.py:61-67)
 //     and its transpose (input gradient: dx+ = Wr^T dy+ + Wi^T dy-,
 //     dx- = -Wi^T dy+ + Wr^T dy-) negate a register copy of Wi.
+// The weights are the MFMA's A operand and the rows its B operand, so an
+// accumulator lane holds one edge (lane & 31) and 16 consecutive channels of
+// the block (half h = lane >> 5: channels 16 h + i in register i; the weight
+// fragment's lanes are read through a permutation that makes them consecutive).
+// Everything that is per edge in the epilogue is then per lane: its kept Wigner
+// entries, its saved rows, radial scales and gate rows are 16-byte loads and
+// stores of the lane's own edge, with no transposition through LDS.  (With lane =
+// channel those went through LDS, edge by edge: 45 000 edges, lmax 6, 128 channels,
+// bf16, gated 1105 us forward and 1087 input gradient, so 1023 and 1038.)
 // Epilogue per owned degree l: [bias, gate | radial scale and its gradient],
-// then for each pair of output columns (j, j+1) and each 16-edge chunk:
-// v = sum_q D(q, j) acc_q per row (Wigner rows in LDS in a pair-major layout,
-// one 16-byte read per (row, 2 j)), staged through LDS so that lane (c, h)
-// holds column j + h of all 16 rows, then a running sum over the edges in
-// order with uniform control (segment ends from a 64-bit ballot mask); each
-// finished segment is stored once (or to the partials buffer when it is cut
-// by a tile boundary).  Deterministic: fixed summation order, no atomics.
+// then for each pair of output columns (j, j+1) and each 32-edge row tile:
+// v = sum_q D(q, j) acc_q in the lane, written to a per-wave LDS tile
+// [edge][2 columns x 32 channels] and read back with lane = (column, channel);
+// the sum over the edges runs in order with uniform control (segment ends from
+// a 64-bit ballot mask); each finished segment is stored once (or to the
+// partials buffer when it is cut by a tile boundary).  Deterministic: fixed
+// summation order, no atomics.
 #include "message_impl.h"
 
 namespace maloq {
@@ -160,17 +169,12 @@ struct GPlan {
     for (int w = 0; w < NW; ++w) m = tab.nslots[w] > m ? tab.nslots[w] : m;
     return m;
   }();
-  // Wigner rows in LDS: the pair-major layout of the dk workspace
+  // Wigner rows: the pair-major layout of the dk workspace
   static constexpr int pblk(int l) { return PairLayout<L, M>::pblk(l); }
   static constexpr int woff(int l) { return PairLayout<L, M>::woff(l); }
   static constexpr int WS = PairLayout<L, M>::WS;
-  // Wigner rows in LDS: TE WS / 4 16-byte chunks, copied by DMA in whole
-  // 64-lane instructions (the array is padded to a multiple of 64 chunks)
-  static constexpr int W16 = TE * WS / 4;
-  static constexpr int W16P = (W16 + 63) / 64 * 64;
   // LDS
   static constexpr int A_BYTES = nqa(L) * RT * FRAG;     // one A stage
-  static constexpr int CH = 16;                           // edges per epilogue chunk
   static constexpr int NA = (nqa(L) * RT * 64 + NT - 1) / NT;  // A chunks per thread
 };
 
@@ -180,14 +184,24 @@ typedef unsigned int frag_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ frag_t neg_frag(frag_t v, BF16) { return v ^ 0x80008000u; }
 __device__ __forceinline__ frag_t neg_frag(frag_t v, F32) { return v ^ 0x80000000u; }
-__device__ __forceinline__ void mfma(f32x16& acc, frag_t a, frag_t b, BF16) {
-  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16((bf16x8)a, (bf16x8)b, acc, 0, 0, 0);
+// acc += (weight fragment w)^T (row fragment a): accumulator rows are output
+// channels, columns (lanes) edges.
+__device__ __forceinline__ void mfma(f32x16& acc, frag_t a, frag_t w, BF16) {
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16((bf16x8)w, (bf16x8)a, acc, 0, 0, 0);
 }
-__device__ __forceinline__ void mfma(f32x16& acc, frag_t a, frag_t b, F32) {
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.x), __uint_as_float(b.x), acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.y), __uint_as_float(b.y), acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.z), __uint_as_float(b.z), acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.w), __uint_as_float(b.w), acc, 0, 0, 0);
+__device__ __forceinline__ void mfma(f32x16& acc, frag_t a, frag_t w, F32) {
+  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(w.x), __uint_as_float(a.x), acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(w.y), __uint_as_float(a.y), acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(w.z), __uint_as_float(a.z), acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(w.w), __uint_as_float(a.w), acc, 0, 0, 0);
+}
+
+// Byte offset in a packed weight fragment (lane i: column i & 31) that lane
+// `lane` reads: accumulator row r = 8 a + 4 h + b then holds channel 16 h + 4 a + b,
+// so register 4 a + b of a lane of half h is channel 16 h + 4 a + b.
+__device__ __forceinline__ int weight_lane(int lane) {
+  const int r = lane & 31;
+  return ((lane & 32) + 16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3)) * 16;
 }
 
 template <int L, int M, bool GATE, int NW, int RT, class TM, int MODE>
@@ -204,9 +218,10 @@ struct Gemm {
   // A stages (three distinct LDS objects, so the compiler can tell a stage
   // being filled by DMA from the one being read); after the K loop they hold
   // the epilogue's per-wave staging, WPS waves per stage (2 of 4 waves: st0
-  // and st1; 3 of 8 waves: all three).
-  // per-wave epilogue staging: the 16-edge scan chunk or the 32 x 36 transpose tile
-  static constexpr int PW = (P::CH * 64 > 32 * 36 ? P::CH * 64 : 32 * 36) * 4;
+  // and st1; 3 of 8 waves: all three): 32 edges x 64 floats, padded to 68 (16-byte
+  // rows; the writes of 8 lanes and the reads of a row are free of bank conflicts).
+  static constexpr int TP = 68;
+  static constexpr int PW = 32 * TP * 4;
   static constexpr int WPS = (NW + 2) / 3;
   // Gate wave (P::GW): after the K loop the stages also carry tanh of the gate
   // rows to the degree waves, degree l's RT x 16 x 64 floats in stage (l - 1) / GPS.
@@ -305,7 +320,7 @@ struct Gemm {
   template <int W, int LI>
   static __device__ __forceinline__ void b_load(frag_t (&b)[P::NBW], const char* wp, int64_t foff,
                                                 int ks, int lane) {
-    const char* base = wp + (foff + static_cast<int64_t>(ks) * P::nbfrag(LI)) * FRAG + lane * 16;
+    const char* base = wp + (foff + static_cast<int64_t>(ks) * P::nbfrag(LI)) * FRAG + weight_lane(lane);
     static_for<L + 1>([&](auto LO) {
       constexpr int lo = decltype(LO)::value;
       if constexpr (P::tab.owner[lo] == W) {
@@ -494,77 +509,81 @@ struct Gemm {
   }
 
   // ------------------------------------------------------------ epilogue
-  // Row of register i in row tile rt for lane half h (32x32 accumulator layout).
-  static __device__ __forceinline__ int row_of(int rt, int i, int h) {
-    return rt * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
+  // In the accumulators lane (co = lane & 31, h = lane >> 5) holds edge co of the
+  // row tile and channels cb CB + 16 h + i, i = 0..15.
+  static __device__ __forceinline__ void load16(const typename TM::raw* p, float (&v)[16]) {
+    float t[8];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      load_vec<TM, 8>(p + 8 * k, t);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[8 * k + i] = t[i];
+    }
+  }
+  static __device__ __forceinline__ void store16(typename TM::raw* p, const float (&v)[16]) {
+    float t[8];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) t[i] = v[8 * k + i];
+      store_vec<TM, 8>(p + 8 * k, t);
+    }
+  }
+  static __device__ __forceinline__ void store16(typename TM::raw* p, const f32x16& v) {
+    float t[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) t[i] = v[i];
+    store16(p, t);
+  }
+  static __device__ __forceinline__ void load_bias(const float* bias, int64_t at, float (&b)[16]) {
+    // branch-free: a runtime branch around accumulator updates costs spills
+#pragma unroll
+    for (int i = 0; i < 16; ++i) b[i] = bias != nullptr ? bias[at + i] : 0.f;
   }
 
+  // col: the lane's first channel
   template <int lo>
   static __device__ __forceinline__ void add_bias(f32x16 (&acc)[P::MSLOT], const Args& a, int col) {
+    float b0[16];
+    load_bias(a.bias, a.extra + static_cast<int64_t>(lo) * a.C_n + col, b0);
     static_for<RT>([&](auto RTI) {
       constexpr int sb = P::tab.base[lo] + decltype(RTI)::value * P::ntype(lo);
-      // branch-free: a runtime branch around accumulator updates costs spills
-      const float b0 = a.bias != nullptr ? a.bias[a.extra + lo * a.C_n + col] : 0.f;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[sb][i] += b0;
-      if constexpr (P::gacc(lo)) {
-        const float bg = a.bias != nullptr ? a.bias[(lo - 1) * a.C_n + col] : 0.f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[sb + 1][i] += bg;
-      }
+      for (int i = 0; i < 16; ++i) acc[sb][i] += b0[i];
     });
+    if constexpr (P::gacc(lo)) {
+      load_bias(a.bias, static_cast<int64_t>(lo - 1) * a.C_n + col, b0);
+      static_for<RT>([&](auto RTI) {
+        constexpr int sb = P::tab.base[lo] + decltype(RTI)::value * P::ntype(lo);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[sb + 1][i] += b0[i];
+      });
+    }
   }
 
   // Gated forward: the pre-activation rows of degree lo (kept rows and the gate
-  // row) to a.gsave [edge id][d' + L][C_n], each 32 x 32 block transposed
-  // through the wave's LDS tile so that a lane stores 16 channels of one edge.
-  // ZOUT: the activated kept rows (no gate rows) to a.zout [edge id][d'][C_n]
-  // instead (the edge-frame output of FWD_EDGE).
+  // row) to a.gsave [edge id][d' + L][C_n].  ZOUT: the activated kept rows (no
+  // gate rows) to a.zout [edge id][d'][C_n] instead (the edge-frame output of
+  // FWD_EDGE).
   template <int lo, bool ZOUT = false>
   static __device__ __forceinline__ void save_pre(const f32x16 (&acc)[P::MSLOT], const Smem& s,
-                                                  const Args& a, int cb, float* tb, int lane) {
-    const int co = lane & 31, h = lane >> 5;
+                                                  const Args& a, int col, int lane) {
     constexpr int RPE = ZOUT ? P::DP : P::DP + L;  // rows per edge of the destination
     static_for<RT>([&](auto RTI) {
       constexpr int rt = decltype(RTI)::value;
       constexpr int sb = P::tab.base[lo] + rt * P::ntype(lo);
-      const int ei = s.eid[rt * 32 + co];
+      const int ei = s.eid[rt * 32 + (lane & 31)];
+      if (ei < 0) return;
       typename TM::raw* g = reinterpret_cast<typename TM::raw*>(ZOUT ? a.zout : a.gsave) +
-                            static_cast<int64_t>(ei >= 0 ? ei : 0) * RPE * a.C_n + cb * CB + 16 * h;
+                            static_cast<int64_t>(ei) * RPE * a.C_n + col;
       static_for<P::ntype(lo)>([&](auto TI) {
         constexpr int t = decltype(TI)::value;  // accumulator type: 0, [gate], +1, -1, ...
         if constexpr (ZOUT && P::gacc(lo) && t == 1) return;
         constexpr int row = (P::gacc(lo) && t == 1) ? P::DP + lo - 1
                                                     : P::mrow(t == 0 ? 0 : t - P::gacc(lo), lo);
-        store_block(acc[sb + t], g, ei, row, a.C_n, tb, co, h);
+        store16(g + static_cast<int64_t>(row) * a.C_n, acc[sb + t]);
       });
     });
-  }
-
-  // One 32-edge x 32-channel accumulator block v to row `row` of each edge's
-  // destination rows g (lane (co, h): edge co, channels 16h..16h+15; nothing
-  // for ei < 0), transposed through the wave's LDS tile tb.
-  static __device__ __forceinline__ void store_block(const f32x16& v, typename TM::raw* g, int ei, int row,
-                                                     int64_t C_n, float* tb, int co, int h) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) tb[tsw(8 * (i >> 2) + 4 * h + (i & 3), co)] = v[i];
-    wave_sync();
-    if (ei >= 0) {
-      float w[16];
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const float4 t4 = *reinterpret_cast<const float4*>(tb + tsw(co, 16 * h + 4 * g4));
-        w[4 * g4] = t4.x; w[4 * g4 + 1] = t4.y; w[4 * g4 + 2] = t4.z; w[4 * g4 + 3] = t4.w;
-      }
-      float w8[8];
-#pragma unroll
-      for (int half = 0; half < 2; ++half) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) w8[k] = w[8 * half + k];
-        store_vec<TM, 8>(g + static_cast<int64_t>(row) * C_n + 8 * half, w8);
-      }
-    }
-    wave_sync();
   }
 
   // ---- gate rows apart (P::GW): wave tab.gowner[l] holds the gate row of
@@ -573,27 +592,29 @@ struct Gemm {
   // [edge id][d' + L][C_n], row d' + l - 1.
   template <int W>
   static __device__ __forceinline__ void gate_rows(f32x16 (&acc)[P::MSLOT], const Smem& s, const Args& a,
-                                                   int cb, float* tb, int lane) {
-    const int co = lane & 31, h = lane >> 5, col = cb * CB + co;
+                                                   int col, int lane) {
     static_for<L + 1>([&](auto LO) {
       constexpr int lo = decltype(LO)::value;
       if constexpr (P::gown(W, lo)) {
-        const float bg = a.bias != nullptr ? a.bias[(lo - 1) * a.C_n + col] : 0.f;
+        float bg[16];
+        load_bias(a.bias, static_cast<int64_t>(lo - 1) * a.C_n + col, bg);
         static_for<RT>([&](auto R) {
 #pragma unroll
-          for (int i = 0; i < 16; ++i) acc[P::tab.gbase[lo] + decltype(R)::value][i] += bg;
+          for (int i = 0; i < 16; ++i) acc[P::tab.gbase[lo] + decltype(R)::value][i] += bg[i];
         });
       }
     });
     if (a.gsave == nullptr) return;
     static_for<RT>([&](auto RTI) {
       constexpr int rt = decltype(RTI)::value;
-      const int ei = s.eid[rt * 32 + co];
+      const int ei = s.eid[rt * 32 + (lane & 31)];
+      if (ei < 0) return;
       typename TM::raw* gp = reinterpret_cast<typename TM::raw*>(a.gsave) +
-                             static_cast<int64_t>(ei >= 0 ? ei : 0) * (P::DP + L) * a.C_n + cb * CB + 16 * h;
+                             static_cast<int64_t>(ei) * (P::DP + L) * a.C_n + col;
       static_for<L + 1>([&](auto LO) {
         constexpr int lo = decltype(LO)::value;
-        if constexpr (P::gown(W, lo)) store_block(acc[P::tab.gbase[lo] + rt], gp, ei, P::DP + lo - 1, a.C_n, tb, co, h);
+        if constexpr (P::gown(W, lo))
+          store16(gp + static_cast<int64_t>(P::DP + lo - 1) * a.C_n, acc[P::tab.gbase[lo] + rt]);
       });
     });
   }
@@ -647,86 +668,54 @@ struct Gemm {
 
   // BWD_EDGE with a.gsave: the GateActivation backward (activation.py:57-77)
   // fused into the edge-frame store.  acc holds o = dL/d(gate output) of degree
-  // lo; after the transpose through LDS a lane holds 16 channels of one edge,
-  // reads the saved pre-activations z of the same row (and the gate row) and
-  // writes to a.zout [edge id][d' + L][C_n]:
+  // lo; a lane reads the saved pre-activations z of the same edge and channels
+  // (and the gate row) and writes to a.zout [edge id][d' + L][C_n]:
   //   lo = 0:  dpre = o s (1 + z (1 - s)),  s = sigmoid(z);
   //   lo >= 1: t = tanh(z_gate); dpre_q = o_q t;  dgate = (1 - t^2) sum_q o_q z_q.
   template <int lo>
   static __device__ __forceinline__ void store_gate_bwd(const f32x16 (&acc)[P::MSLOT], const Smem& s,
-                                                        const Args& a, int cb, float* tb, int lane) {
+                                                        const Args& a, int col, int lane) {
     constexpr int DG = P::DP + L;
-    const int co = lane & 31, h = lane >> 5;
     static_for<RT>([&](auto RTI) {
       constexpr int rt = decltype(RTI)::value;
       constexpr int sb = P::tab.base[lo] + rt * P::ntype(lo);
-      const int ei = s.eid[rt * 32 + co];
-      const int64_t base = static_cast<int64_t>(ei >= 0 ? ei : 0) * DG * a.C_n + cb * CB + 16 * h;
+      const int ei = s.eid[rt * 32 + (lane & 31)];
+      if (ei < 0) return;
+      const int64_t base = static_cast<int64_t>(ei) * DG * a.C_n + col;
       typename TM::raw* g = reinterpret_cast<typename TM::raw*>(a.zout) + base;
       const typename TM::raw* zs = reinterpret_cast<const typename TM::raw*>(a.gsave) + base;
-      float tg[16], dg[16];
-      if constexpr (lo > 0) {
+      float z[16], w[16];
+      if constexpr (lo == 0) {
+        load16(zs + static_cast<int64_t>(P::mrow(0, 0)) * a.C_n, z);
 #pragma unroll
-        for (int k = 0; k < 16; ++k) {
-          tg[k] = 0.f;
-          dg[k] = 0.f;
+        for (int i = 0; i < 16; ++i) {
+          const float sg = 1.0f / (1.0f + expf(-z[i]));
+          w[i] = acc[sb][i] * (sg * (1.0f + z[i] * (1.0f - sg)));
         }
-        if (ei >= 0) {
-          float t8[8];
+        store16(g + static_cast<int64_t>(P::mrow(0, 0)) * a.C_n, w);
+      } else {
+        float tg[16], dg[16];
+        load16(zs + static_cast<int64_t>(P::DP + lo - 1) * a.C_n, tg);
 #pragma unroll
-          for (int half = 0; half < 2; ++half) {
-            load_vec<TM, 8>(zs + static_cast<int64_t>(P::DP + lo - 1) * a.C_n + 8 * half, t8);
-#pragma unroll
-            for (int k = 0; k < 8; ++k) tg[8 * half + k] = tanhf(t8[k]);
-          }
+        for (int i = 0; i < 16; ++i) {
+          tg[i] = tanhf(tg[i]);
+          dg[i] = 0.f;
         }
-      }
-      static_for<P::ntype(lo)>([&](auto TI) {
-        constexpr int t = decltype(TI)::value;
-        constexpr int row = P::mrow(t, lo);
+        static_for<P::ntype(lo)>([&](auto TI) {
+          constexpr int t = decltype(TI)::value;
+          constexpr int row = P::mrow(t, lo);
+          load16(zs + static_cast<int64_t>(row) * a.C_n, z);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) tb[tsw(8 * (i >> 2) + 4 * h + (i & 3), co)] = acc[sb + t][i];
-        wave_sync();
-        if (ei >= 0) {
-          float v[16];
-#pragma unroll
-          for (int g4 = 0; g4 < 4; ++g4) {
-            const float4 t4 = *reinterpret_cast<const float4*>(tb + tsw(co, 16 * h + 4 * g4));
-            v[4 * g4] = t4.x; v[4 * g4 + 1] = t4.y; v[4 * g4 + 2] = t4.z; v[4 * g4 + 3] = t4.w;
+          for (int i = 0; i < 16; ++i) {
+            const float o = acc[sb + t][i];
+            dg[i] = fmaf(o, z[i], dg[i]);
+            w[i] = o * tg[i];
           }
+          store16(g + static_cast<int64_t>(row) * a.C_n, w);
+        });
 #pragma unroll
-          for (int half = 0; half < 2; ++half) {
-            float z8[8], w8[8];
-            load_vec<TM, 8>(zs + static_cast<int64_t>(row) * a.C_n + 8 * half, z8);
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-              const float o = v[8 * half + k], z = z8[k];
-              if constexpr (lo == 0) {
-                const float sg = 1.0f / (1.0f + expf(-z));
-                w8[k] = o * (sg * (1.0f + z * (1.0f - sg)));
-              } else {
-                dg[8 * half + k] = fmaf(o, z, dg[8 * half + k]);
-                w8[k] = o * tg[8 * half + k];
-              }
-            }
-            store_vec<TM, 8>(g + static_cast<int64_t>(row) * a.C_n + 8 * half, w8);
-          }
-        }
-        wave_sync();
-      });
-      if constexpr (lo > 0) {
-        if (ei >= 0) {
-#pragma unroll
-          for (int half = 0; half < 2; ++half) {
-            float w8[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-              const float tv = tg[8 * half + k];
-              w8[k] = dg[8 * half + k] * (1.0f - tv * tv);
-            }
-            store_vec<TM, 8>(g + static_cast<int64_t>(P::DP + lo - 1) * a.C_n + 8 * half, w8);
-          }
-        }
+        for (int i = 0; i < 16; ++i) w[i] = dg[i] * (1.0f - tg[i] * tg[i]);
+        store16(g + static_cast<int64_t>(P::DP + lo - 1) * a.C_n, w);
       }
     });
   }
@@ -758,173 +747,127 @@ struct Gemm {
 
   // Input gradient: the accumulators hold dY (forward-input side) of degree lo.
   // grad_rad = sum_(+-) dY * R (R: unscaled forward rows); dY *= rad.
-  // Each 32-edge x 32-channel block of dY is transposed through a per-wave
-  // LDS tile (pitch 36 floats: 16-byte rows, at most 2-way bank conflicts) into row layout, where lane (edge r,
-  // half h) holds channels 16h..16h+15 of one edge: R, rad and grad_rad then
-  // move as 32- or 64-byte vectors per lane; the scaled block is transposed
-  // back for the inverse rotation.
-  static __device__ __forceinline__ int tsw(int r, int c) { return r * 36 + c; }
-
   template <int lo>
   static __device__ __forceinline__ void radial(f32x16 (&acc)[P::MSLOT], const Smem& s,
-                                                const Args& a, int cb, float* tb, int lane) {
+                                                const Args& a, int col, int lane) {
     const int64_t rw = rad_width<L, M>(a.C_n);
-    const int co = lane & 31, h = lane >> 5;
-    const int c0 = cb * CB + h * 16;  // first channel of this lane in row layout
-    constexpr int VEC = TM::VEC;      // channels per 16-byte piece
-    constexpr int NU = 16 / VEC;      // 16-byte pieces per 16 channels
     static_for<RT>([&](auto RTI) {
       constexpr int rt = decltype(RTI)::value;
       constexpr int sb = P::tab.base[lo] + rt * P::ntype(lo);
-      const int ei = s.eid[rt * 32 + co];
+      const int ei = s.eid[rt * 32 + (lane & 31)];
       const int64_t eis = ei >= 0 ? ei : s.eid[0];
       const typename TM::raw* rsave = reinterpret_cast<const typename TM::raw*>(a.rsave) +
-                                      eis * P::DP * a.C_n + c0;
+                                      eis * P::DP * a.C_n + col;
       static_for<1 + (lo < M ? lo : M)>([&](auto MI) {
         constexpr int m = decltype(MI)::value;
         constexpr int q0 = m == 0 ? 0 : 2 * m - 1, nqm = m == 0 ? 1 : 2;
-        const typename TM::raw* radp = reinterpret_cast<const typename TM::raw*>(a.rad) + eis * rw +
-                                       rad_slot<L, M>(q0, lo, c0, a.C_n);
-        // bf16: this lane's 16 channels of the radial slot, and below of each R
-        // row, issued before the LDS round trips that transpose the block (one
-        // memory latency per block rather than one per 4 channels); fp32 (twice
-        // the registers) loads them where they are used
-        constexpr bool PF = sizeof(typename TM::raw) == 2;
-        uint4 rv_u[NU];
-        if constexpr (PF) {
+        const int64_t slot = rad_slot<L, M>(q0, lo, col, a.C_n);
+        float rv[16], dr[16];
+        load16(reinterpret_cast<const typename TM::raw*>(a.rad) + eis * rw + slot, rv);
 #pragma unroll
-          for (int k = 0; k < NU; ++k) rv_u[k] = reinterpret_cast<const uint4*>(radp)[k];
-        }
-        float dr[16];
-#pragma unroll
-        for (int k = 0; k < 16; ++k) dr[k] = 0.f;
+        for (int i = 0; i < 16; ++i) dr[i] = 0.f;
         static_for<nqm>([&](auto QI) {
           constexpr int q = q0 + decltype(QI)::value;
-          constexpr int slot = sb + P::qtype(q, lo);
-          __builtin_amdgcn_sched_barrier(0);  // one block at a time (register pressure)
-          uint4 rr_u[NU];
-          if constexpr (PF) {
+          constexpr int sl = sb + P::qtype(q, lo);
+          float rr[16];
+          load16(rsave + static_cast<int64_t>(P::mrow(q, lo)) * a.C_n, rr);
 #pragma unroll
-            for (int k = 0; k < NU; ++k) rr_u[k] = reinterpret_cast<const uint4*>(rsave + P::mrow(q, lo) * a.C_n)[k];
+          for (int i = 0; i < 16; ++i) {
+            dr[i] = fmaf(acc[sl][i], rr[i], dr[i]);
+            acc[sl][i] *= rv[i];
           }
-          // accumulator layout -> row layout
-#pragma unroll
-          for (int i = 0; i < 16; ++i) tb[tsw(8 * (i >> 2) + 4 * h + (i & 3), co)] = acc[slot][i];
-          wave_sync();
-#pragma unroll
-          for (int g = 0; g < NU; ++g) {  // VEC channels at a time
-            float rr[VEC], rv[VEC];
-            if constexpr (PF) {
-              unpack_vec<TM, VEC>(rr_u[g], rr);
-              unpack_vec<TM, VEC>(rv_u[g], rv);
-            } else {
-              unpack_vec<TM, VEC>(reinterpret_cast<const uint4*>(rsave + P::mrow(q, lo) * a.C_n)[g], rr);
-              unpack_vec<TM, VEC>(reinterpret_cast<const uint4*>(radp)[g], rv);
-            }
-#pragma unroll
-            for (int g4 = 0; g4 < VEC / 4; ++g4) {
-              const int cc = VEC * g + 4 * g4;
-              float4 t4 = *reinterpret_cast<const float4*>(tb + tsw(co, 16 * h + cc));
-              dr[cc] = fmaf(t4.x, rr[4 * g4], dr[cc]);
-              dr[cc + 1] = fmaf(t4.y, rr[4 * g4 + 1], dr[cc + 1]);
-              dr[cc + 2] = fmaf(t4.z, rr[4 * g4 + 2], dr[cc + 2]);
-              dr[cc + 3] = fmaf(t4.w, rr[4 * g4 + 3], dr[cc + 3]);
-              t4.x *= rv[4 * g4]; t4.y *= rv[4 * g4 + 1]; t4.z *= rv[4 * g4 + 2]; t4.w *= rv[4 * g4 + 3];
-              *reinterpret_cast<float4*>(tb + tsw(co, 16 * h + cc)) = t4;
-            }
-          }
-          wave_sync();
-#pragma unroll
-          for (int i = 0; i < 16; ++i) acc[slot][i] = tb[tsw(8 * (i >> 2) + 4 * h + (i & 3), co)];
-          wave_sync();
         });
-        if (a.drad != nullptr && ei >= 0) {
-          typename TM::raw* dp = reinterpret_cast<typename TM::raw*>(a.drad) + ei * rw +
-                                 rad_slot<L, M>(q0, lo, c0, a.C_n);
-          float t[8];
-#pragma unroll
-          for (int half = 0; half < 2; ++half) {
-#pragma unroll
-            for (int k = 0; k < 8; ++k) t[k] = dr[8 * half + k];
-            store_vec<TM, 8>(dp + 8 * half, t);
-          }
-        }
+        if (a.drad != nullptr && ei >= 0)
+          store16(reinterpret_cast<typename TM::raw*>(a.drad) + ei * rw + slot, dr);
+        __builtin_amdgcn_sched_barrier(0);  // one block at a time (register pressure)
       });
     });
   }
 
   // Inverse rotation of degree lo and segment sum into out / partials.
-  // Per output-column pair p (j = 2p + h for lane half h) and 16-edge chunk:
-  // rotate the rows a lane holds (rows of its half), swap halves with
-  // v_permlane32_swap so that each lane holds its column j for all 16 rows,
-  // run a segmented sum in edge order (uniform selects at segment starts),
-  // then store the sums of the segments that end in the chunk.
+  // Per output-column pair p (j = 2p, 2p + 1) and row tile: rotate the lane's
+  // edge (its Wigner entries straight from the dk rows, one pair ahead), write
+  // both columns to the wave's LDS tile [edge][column][channel], read them back
+  // with lane (channel, column) = (lane & 31, lane >> 5), sum over the edges in
+  // order, and store the sums of the segments that end in the tile.
   template <int W, int lo>
-  static __device__ __forceinline__ void rotate_sum(f32x16 (&acc)[P::MSLOT], Smem& s,
-                                                    const float* wsh, const Args& a, int cb,
+  static __device__ __forceinline__ void rotate_sum(f32x16 (&acc)[P::MSLOT], Smem& s, const Args& a, int cb,
                                                     float* buf, int lane, uint64_t endmask) {
     constexpr int n = 2 * lo + 1;
     constexpr int nq = P::nq(lo);
     constexpr int PB = P::pblk(lo);
     const int co = lane & 31, h = lane >> 5;
-    const float* Wl = wsh + P::woff(lo);
-    const uint64_t startmask = (endmask << 1) | 1ull;
+    const int ow = a.ow > 0 ? a.ow : a.C_n;
+    const int ocb = a.ow > 0 ? cb - a.cb0 : cb;
+    const float4* Dp[RT];
+    static_for<RT>([&](auto R) {
+      constexpr int rt = decltype(R)::value;
+      const int e = s.eid[rt * 32 + co] >= 0 ? s.eid[rt * 32 + co] : s.eid[0];
+      Dp[rt] = reinterpret_cast<const float4*>(a.dk + static_cast<int64_t>(e) * P::WS + P::woff(lo));
+    });
+    float4 nxt[PB / 4];
+#pragma unroll
+    for (int v = 0; v < PB / 4; ++v) nxt[v] = Dp[0][v];
+    float* wr = buf + co * TP + 16 * h;
+    const float* rd = buf + lane;
     for (int p = 0; p <= lo; ++p) {
       const bool has_col = 2 * p + h < n;
-      const int ow = a.ow > 0 ? a.ow : a.C_n;
-      const int ocb = a.ow > 0 ? cb - a.cb0 : cb;
       const int64_t colo = static_cast<int64_t>(lo * lo + 2 * p + h) * ow + ocb * CB + co;
       float run = 0.f;
-      static_for<2 * RT>([&](auto CI) {
-        constexpr int c = decltype(CI)::value;
-        constexpr int rt = c / 2, ib = 8 * (c % 2);
+      static_for<RT>([&](auto R) {
+        constexpr int rt = decltype(R)::value;
         constexpr int sb = P::tab.base[lo] + rt * P::ntype(lo);
-        float X[8], Y[8];
+        float dv[PB];
 #pragma unroll
-        for (int ii = 0; ii < 8; ++ii) {
-          const int i = ib + ii;
-          const int e = row_of(rt, i, h);
-          const float4* Dp = reinterpret_cast<const float4*>(Wl + e * P::WS + p * PB);
-          float dv[PB];
-#pragma unroll
-          for (int v = 0; v < PB / 4; ++v) {
-            const float4 t4 = Dp[v];
-            dv[4 * v] = t4.x; dv[4 * v + 1] = t4.y; dv[4 * v + 2] = t4.z; dv[4 * v + 3] = t4.w;
-          }
-          float v0 = 0.f, v1 = 0.f;
-          static_for<nq>([&](auto Q) {
-            constexpr int q = decltype(Q)::value;
-            const float z = acc[sb + P::qtype(q, lo)][i];
-            v0 = fmaf(dv[2 * q], z, v0);
-            v1 = fmaf(dv[2 * q + 1], z, v1);
-          });
-          // lanes 32-63 of v0 <-> lanes 0-31 of v1: afterwards lane (co, h) holds
-          // column 2p + h, rows of half 0 in v0 and rows of half 1 in v1
-          const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(v0), __float_as_uint(v1),
-                                                           false, false);
-          X[ii] = __uint_as_float(sw[0]);
-          Y[ii] = __uint_as_float(sw[1]);
+        for (int v = 0; v < PB / 4; ++v) {
+          dv[4 * v] = nxt[v].x; dv[4 * v + 1] = nxt[v].y; dv[4 * v + 2] = nxt[v].z; dv[4 * v + 3] = nxt[v].w;
         }
-        // chunk rows in edge order: X[0..3], Y[0..3], X[4..7], Y[4..7].  The
-        // chunk's segment starts, opaque per chunk: otherwise the compiler
-        // hoists all 64 uniform selects out of the column loop and spills them.
-        uint32_t sm = static_cast<uint32_t>(startmask >> (c * P::CH)) & 0xffffu;
-        asm volatile("" : "+s"(sm));
-        static_for<P::CH>([&](auto UI) {
-          constexpr int u = decltype(UI)::value;
-          constexpr int k = 4 * (u >> 3) + (u & 3);
-          const float val = ((u >> 2) & 1) ? Y[k] : X[k];
-          run = ((sm >> u) & 1u) ? val : run + val;
-          buf[u * 64 + lane] = run;
-        });
+        {
+          const int np = rt + 1 < RT ? p : (p < lo ? p + 1 : lo);
+          constexpr int nrt = rt + 1 < RT ? rt + 1 : 0;
+#pragma unroll
+          for (int v = 0; v < PB / 4; ++v) nxt[v] = Dp[nrt][np * (PB / 4) + v];
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            float o[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              o[k] = 0.f;
+              static_for<nq>([&](auto Q) {
+                constexpr int q = decltype(Q)::value;
+                o[k] = fmaf(dv[2 * q + j], acc[sb + P::qtype(q, lo)][4 * g + k], o[k]);
+              });
+            }
+            *reinterpret_cast<float4*>(wr + 32 * j + 4 * g) = make_float4(o[0], o[1], o[2], o[3]);
+          }
         wave_sync();
-        uint32_t m = static_cast<uint32_t>(endmask >> (c * P::CH)) & 0xffffu;
-        while (m) {
-          const int u = __builtin_ctz(m);
-          m &= m - 1u;
-          const float v = buf[u * 64 + lane];
-          float* dst = s.optr[c * P::CH + u];
-          if (has_col) dst[colo] = v;
+        // the tile's segment ends, opaque per tile: otherwise the compiler hoists
+        // the uniform branches' conditions out of the column loop and spills them
+        uint32_t em = static_cast<uint32_t>(endmask >> (32 * rt));
+        asm volatile("" : "+s"(em));
+        float x[32];
+#pragma unroll
+        for (int u = 0; u < 32; ++u) x[u] = rd[u * TP];
+#pragma unroll
+        for (int u = 0; u < 32; u += 4) {
+          if (((em >> u) & 15u) == 0u) {
+            run += x[u];
+            run += x[u + 1];
+            run += x[u + 2];
+            run += x[u + 3];
+          } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              run += x[u + k];
+              if ((em >> (u + k)) & 1u) {
+                if (has_col) s.optr[rt * 32 + u + k][colo] = run;
+                run = 0.f;
+              }
+            }
+          }
         }
         wave_sync();
       });
@@ -932,7 +875,7 @@ struct Gemm {
   }
 
   template <int W, int KR, bool RAD>
-  static __device__ __forceinline__ void body(Smem& s, const float* wsh, char* st0, char* st1, char* st2,
+  static __device__ __forceinline__ void body(Smem& s, char* st0, char* st1, char* st2,
                                               const Args& a,
                                               int cb, int tid, int nvalid) {
     const int wave = tid >> 6, lane = tid & 63;
@@ -967,7 +910,7 @@ struct Gemm {
     // segment ends of the tile: bit e set if edge e closes its segment
     const int le = lane < TE ? lane : TE - 1, ln = le + 1 < TE ? le + 1 : le;
     const uint64_t endmask = __ballot(lane < nvalid && (lane == nvalid - 1 || s.seg[ln] != s.seg[le]));
-    const int col = cb * CB + (lane & 31);
+    const int col = cb * CB + 16 * (lane >> 5);  // the lane's first channel
     if constexpr (P::GW) {
       // bias and pre-activation rows; the gate values through the stages (every
       // wave passes the three barriers); the activation; the stores
@@ -976,11 +919,10 @@ struct Gemm {
         constexpr int lo = decltype(LO)::value;
         if constexpr (P::tab.owner[lo] == W) {
           add_bias<lo>(acc, a, col);
-          if (a.gsave != nullptr) save_pre<lo>(acc, s, a, cb, tb, lane);
+          if (a.gsave != nullptr) save_pre<lo>(acc, s, a, col, lane);
         }
       });
-      gate_rows<W>(acc, s, a, cb, tb, lane);
-      __syncthreads();  // staging reads done before the gate values overwrite it
+      gate_rows<W>(acc, s, a, col, lane);
       gate_out<W>(acc, st0, st1, st2, lane);
       __syncthreads();
       static_for<L + 1>([&](auto LO) {
@@ -992,9 +934,9 @@ struct Gemm {
         constexpr int lo = decltype(LO)::value;
         if constexpr (P::tab.owner[lo] == W) {
           if constexpr (MODE == FWD_EDGE)
-            save_pre<lo, true>(acc, s, a, cb, tb, lane);
+            save_pre<lo, true>(acc, s, a, col, lane);
           else
-            rotate_sum<W, lo>(acc, s, wsh, a, cb, tb, lane, endmask);
+            rotate_sum<W, lo>(acc, s, a, cb, tb, lane, endmask);
         }
       });
       return;
@@ -1005,24 +947,17 @@ struct Gemm {
         if constexpr (!P::BWD) {
           add_bias<lo>(acc, a, col);
           if constexpr (GATE) {
-            if (a.gsave != nullptr)
-              save_pre<lo>(acc, s, a, cb,
-                           wave_staging(wave, st0, st1, st2), lane);
+            if (a.gsave != nullptr) save_pre<lo>(acc, s, a, col, lane);
             gate_act<lo>(acc);
           }
         } else if constexpr (RAD)
-          radial<lo>(acc, s, a, cb,
-                     wave_staging(wave, st0, st1, st2), lane);
+          radial<lo>(acc, s, a, col, lane);
         if constexpr (MODE == BWD_EDGE)
-          store_gate_bwd<lo>(acc, s, a, cb,
-                             wave_staging(wave, st0, st1, st2), lane);
+          store_gate_bwd<lo>(acc, s, a, col, lane);
         else if constexpr (MODE == FWD_EDGE)
-          save_pre<lo, true>(acc, s, a, cb,
-                             wave_staging(wave, st0, st1, st2), lane);
+          save_pre<lo, true>(acc, s, a, col, lane);
         else
-          rotate_sum<W, lo>(acc, s, wsh, a, cb,
-                            wave_staging(wave, st0, st1, st2),
-                            lane, endmask);
+          rotate_sum<W, lo>(acc, s, a, cb, wave_staging(wave, st0, st1, st2), lane, endmask);
       }
     });
   }
@@ -1033,9 +968,6 @@ struct Gemm {
     __shared__ alignas(16) char st0[SB];
     __shared__ alignas(16) char st1[SB];
     __shared__ alignas(16) char st2[SB];
-    // Wigner rows of the tile: its own LDS object, so that the compiler can tell
-    // its DMA apart from the accesses to s
-    __shared__ alignas(16) float wsh[P::W16P * 4];
     const int tid = threadIdx.x, wave = tid >> 6;
     // XCD-aware mapping: consecutive workgroup ids go round-robin over the 8
     // XCDs.  The n_cb channel-block workgroups of one edge tile are the
@@ -1073,32 +1005,9 @@ struct Gemm {
       }
       s.optr[tid] = dst;
     }
-    // Wigner rows of the tile's edges (pair layout): DMA straight into LDS,
-    // issued after every global load whose value the prologue waits for, so it
-    // is in flight with the first K steps; the K loop's waits and barriers
-    // complete it long before the epilogue reads it.  Chunk i = 64 (k NW + w) +
-    // lane is instruction k of wave w; lanes past the tile read an in-bounds row
-    // into the padding; rows of edges past the tile are never stored.
-    // FWD_EDGE and BWD_EDGE do not rotate back: no rows.
-    if constexpr (MODE != FWD_EDGE && MODE != BWD_EDGE) {
-      constexpr int R4 = P::WS / 4;
-      const float4* dk4 = reinterpret_cast<const float4*>(a.dk);
-      const int wv = __builtin_amdgcn_readfirstlane(wave), lane = tid & 63;
-      for (int k = 0; k < (P::W16P / 64 + NW - 1) / NW; ++k) {
-        const int blk = k * NW + wv;  // uniform
-        if (blk >= P::W16P / 64) break;
-        const int i = blk * 64 + lane;
-        const int e = i / R4 < TE ? i / R4 : TE - 1;
-        const int ei = s.eid[e] >= 0 ? s.eid[e] : s.eid[0];
-#if defined(__HIP_DEVICE_COMPILE__)
-        __builtin_amdgcn_global_load_lds(dk4 + static_cast<int64_t>(ei) * R4 + (i - (i / R4) * R4),
-                                         (lds_void*)(reinterpret_cast<char*>(wsh) + blk * 1024), 16, 0, 0);
-#endif
-      }
-    }
     static_for<NW>([&](auto WI) {
       constexpr int w = decltype(WI)::value;
-      if (wave == w) body<w, KR, RAD>(s, wsh, st0, st1, st2, a, cb, tid, nvalid);
+      if (wave == w) body<w, KR, RAD>(s, st0, st1, st2, a, cb, tid, nvalid);
     });
   }
 };
