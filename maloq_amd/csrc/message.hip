@@ -167,14 +167,14 @@ extern "C" int maloq_message_fwd(int dtype, int lmax, int mmax, int gate, const 
     a.wpack = static_cast<const char*>(wpack); a.bias = bias; a.out = out;
     a.part = partials; a.E = num_edges; a.C_k = c_in; a.C_n = c_out; a.n_cb = c_out / CB;
     a.extra = gate ? lmax * c_out : 0;
-    a.ntiles = (num_edges + tile_edges(lmax, mmax, gate) - 1) / tile_edges(lmax, mmax, gate);
+    a.ntiles = (num_edges + tile_edges(dtype, lmax, mmax, gate) - 1) / tile_edges(dtype, lmax, mmax, gate);
     const int kc = dtype == 1 ? BF16::KC : F32::KC;
     a.frags_per_cb = frags_per_cb(lmax, mmax, gate, c_in, kc);
     a.gsave = gate ? gate_ws : nullptr;
     rc = dispatch(lmax, mmax, dtype, gate, FWD, a, s);
     if (rc) return rc;
   }
-  return fixup(seg_ptr, num_nodes, partials, out, d * c_out, tile_edges(lmax, mmax, gate), s);
+  return fixup(seg_ptr, num_nodes, partials, out, d * c_out, tile_edges(dtype, lmax, mmax, gate), s);
 }
 
 // ------------------------------------------------- forward without allocation
@@ -275,7 +275,7 @@ extern "C" int maloq_message_edgewise_fwd(int dtype, int lmax, int mmax, const v
     a.wpack = static_cast<const char*>(wpack1); a.bias = bias1; a.out = out; a.part = partials;
     a.E = num_edges; a.C_k = parts * c_x; a.C_n = c_hidden; a.n_cb = c_hidden / CB;
     a.extra = lmax * c_hidden;
-    a.ntiles = (num_edges + tile_edges(lmax, mmax, 1, FWD_EDGE) - 1) / tile_edges(lmax, mmax, 1, FWD_EDGE);
+    a.ntiles = (num_edges + tile_edges(dtype, lmax, mmax, 1, FWD_EDGE) - 1) / tile_edges(dtype, lmax, mmax, 1, FWD_EDGE);
     a.frags_per_cb = frags_per_cb(lmax, mmax, 1, parts * c_x, kc);
     a.gsave = gate_ws; a.zout = z_ws;
     rc = dispatch(lmax, mmax, dtype, 1, FWD_EDGE, a, s);
@@ -285,12 +285,12 @@ extern "C" int maloq_message_edgewise_fwd(int dtype, int lmax, int mmax, const v
     b.a_src = z_ws; b.dk = dk_ws; b.seg = seg; b.eidx = nullptr;
     b.wpack = static_cast<const char*>(wpack2); b.bias = bias2; b.out = out; b.part = partials;
     b.E = num_edges; b.C_k = c_hidden; b.C_n = c_out; b.n_cb = c_out / CB; b.extra = 0;
-    b.ntiles = (num_edges + tile_edges(lmax, mmax, 0) - 1) / tile_edges(lmax, mmax, 0);
+    b.ntiles = (num_edges + tile_edges(dtype, lmax, mmax, 0) - 1) / tile_edges(dtype, lmax, mmax, 0);
     b.frags_per_cb = frags_per_cb(lmax, mmax, 0, c_hidden, kc);
     rc = dispatch(lmax, mmax, dtype, 0, FWD, b, s);
     if (rc) return rc;
   }
-  return fixup(seg_ptr, num_nodes, partials, out, d * c_out, tile_edges(lmax, mmax, 0), s);
+  return fixup(seg_ptr, num_nodes, partials, out, d * c_out, tile_edges(dtype, lmax, mmax, 0), s);
 }
 
 extern "C" int maloq_message_edgewise_bwd_dx(
@@ -329,7 +329,7 @@ extern "C" int maloq_message_edgewise_bwd_dx(
     b.a_src = dz2_ws; b.dk = dk; b.seg = dst; b.eidx = nullptr;
     b.wpack = static_cast<const char*>(wpack2_t); b.out = grad_x_src; b.part = partials;
     b.E = num_edges; b.C_k = c_x; b.C_n = c_hidden; b.n_cb = c_hidden / CB;
-    b.ntiles = (num_edges + tile_edges(lmax, mmax, 0) - 1) / tile_edges(lmax, mmax, 0);
+    b.ntiles = (num_edges + tile_edges(dtype, lmax, mmax, 0) - 1) / tile_edges(dtype, lmax, mmax, 0);
     b.frags_per_cb = frags_per_cb(lmax, mmax, 0, c_x, kc);
     b.zout = dz1_ws; b.gsave = const_cast<void*>(gate_saved);
     rc = dispatch(lmax, mmax, dtype, 0, BWD_EDGE, b, s);
@@ -347,21 +347,21 @@ extern "C" int maloq_message_edgewise_bwd_dx(
       a.part = partials; a.E = num_edges; a.C_k = c_hidden; a.C_n = parts * c_x;
       a.cb0 = part * (c_x / CB); a.n_cb = c_x / CB;
       a.ow = c_x;   // each part's gradient is its own [*, d, c_x] array
-      a.ntiles = (num_edges + tile_edges(lmax, mmax, 1, BWD_DX) - 1) / tile_edges(lmax, mmax, 1, BWD_DX);
+      a.ntiles = (num_edges + tile_edges(dtype, lmax, mmax, 1, BWD_DX) - 1) / tile_edges(dtype, lmax, mmax, 1, BWD_DX);
       a.frags_per_cb = frags_per_cb(lmax, mmax, 1, c_hidden, kc);
       rc = dispatch(lmax, mmax, dtype, 1, BWD_DX, a, s);
       if (rc) return rc;
       // per-edge rows of the message part: single-edge segments, never cut
       if (part == 2) continue;
       rc = fixup(part ? seg_ptr : seg_ptr_src, num_nodes, partials, part ? grad_x_dst : grad_x_src,
-                 d * c_x, tile_edges(lmax, mmax, 1, BWD_DX), s);
+                 d * c_x, tile_edges(dtype, lmax, mmax, 1, BWD_DX), s);
       if (rc) return rc;
     }
     return MALOQ_OK;
   }
-  rc = fixup(seg_ptr_src, num_nodes, partials, grad_x_src, d * c_x, tile_edges(lmax, mmax, 1, BWD_DX), s);
+  rc = fixup(seg_ptr_src, num_nodes, partials, grad_x_src, d * c_x, tile_edges(dtype, lmax, mmax, 1, BWD_DX), s);
   if (rc) return rc;
-  return fixup(seg_ptr, num_nodes, partials, grad_x_dst, d * c_x, tile_edges(lmax, mmax, 1, BWD_DX), s);
+  return fixup(seg_ptr, num_nodes, partials, grad_x_dst, d * c_x, tile_edges(dtype, lmax, mmax, 1, BWD_DX), s);
 }
 
 extern "C" int maloq_message_bwd_dx(int dtype, int lmax, int mmax, int gate, const float* grad_out,
@@ -397,11 +397,11 @@ extern "C" int maloq_message_bwd_dx(int dtype, int lmax, int mmax, int gate, con
     a.rad = rad; a.drad = grad_rad; a.rsave = r_saved;
     a.wpack = static_cast<const char*>(wpack_t); a.bias = nullptr; a.out = grad_x;
     a.part = partials; a.E = num_edges; a.C_k = c_out; a.C_n = c_in; a.n_cb = c_in / CB;
-    a.extra = 0; a.ntiles = (num_edges + tile_edges(lmax, mmax, gate, BWD_DX) - 1) / tile_edges(lmax, mmax, gate, BWD_DX);
+    a.extra = 0; a.ntiles = (num_edges + tile_edges(dtype, lmax, mmax, gate, BWD_DX) - 1) / tile_edges(dtype, lmax, mmax, gate, BWD_DX);
     const int kc = dtype == 1 ? BF16::KC : F32::KC;
     a.frags_per_cb = frags_per_cb(lmax, mmax, gate, c_out, kc);
     rc = dispatch(lmax, mmax, dtype, gate, BWD_DX, a, s);
     if (rc) return rc;
   }
-  return fixup(seg_ptr_src, num_nodes, partials, grad_x, d * c_in, tile_edges(lmax, mmax, gate, BWD_DX), s);
+  return fixup(seg_ptr_src, num_nodes, partials, grad_x, d * c_in, tile_edges(dtype, lmax, mmax, gate, BWD_DX), s);
 }

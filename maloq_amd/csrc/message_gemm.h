@@ -29,9 +29,7 @@
 // fragment's lanes are read through a permutation that makes them consecutive).
 // Everything that is per edge in the epilogue is then per lane: its kept Wigner
 // entries, its saved rows, radial scales and gate rows are 16-byte loads and
-// stores of the lane's own edge, with no transposition through LDS.  (With lane =
-// channel those went through LDS, edge by edge: 45 000 edges, lmax 6, 128 channels,
-// bf16, gated 1105 us forward and 1087 input gradient, so 1023 and 1038.)
+// stores of the lane's own edge, with no transposition through LDS.
 // Epilogue per owned degree l: [bias, gate | radial scale and its gradient],
 // then for each pair of output columns (j, j+1) and each 32-edge row tile:
 // v = sum_q D(q, j) acc_q in the lane, written to a per-wave LDS tile
@@ -59,12 +57,12 @@ struct GPlan {
   static constexpr int gin(int l) { return (GATE && BWD && l >= 1) ? 1 : 0; }   // input gate row
   static constexpr int nq(int l) { return 1 + 2 * cmin(M, l); }
   static constexpr int nqa(int l) { return nq(l) + gin(l); }  // A row types of input degree l
-  // Gate rows apart (GW): a gated forward on 8 waves (lmax 6) puts the gate
+  // Gate rows apart (GW): a gated forward at lmax 6, mmax < lmax puts the gate
   // row of each degree l >= 1 in the wave with the fewest accumulators at that
   // point (the wave left without a degree, then those of the light degrees),
   // so the waves of the heavy degrees hold only their kept rows; the gate
   // values reach a degree's wave through LDS after the K loop.
-  static constexpr bool GW = GATE && !BWD && NW == 8;
+  static constexpr bool GW = GATE && !BWD && L > 4 && M < L;
   static constexpr int gacc(int l) { return GW ? 0 : gt(l); }  // gate row among degree l's accumulators
   static constexpr int ntype(int l) { return nq(l) + gacc(l); }
   // accumulator type of row type q of degree l (0: m=0, [1: gate], then +1, -1, +2, ...)
@@ -213,7 +211,8 @@ struct Gemm {
   struct Smem {
     float* optr[TE];  // destination row block of the segment ending at each edge
     int seg[TE];
-    int eid[TE];
+    int eid[TE];  // -1 past the tile's edges
+    int safe;     // an edge id that may be read in their place
   };
   // A stages (three distinct LDS objects, so the compiler can tell a stage
   // being filled by DMA from the one being read); after the K loop they hold
@@ -294,7 +293,7 @@ struct Gemm {
       if constexpr (k >= atab.count[W]) return;
       constexpr int rt = afrag<W, k>() % RT;
       const int e = rt * 32 + (lane & 31);
-      const int ei = s.eid[e] >= 0 ? s.eid[e] : s.eid[0];
+      const int ei = s.eid[e] >= 0 ? s.eid[e] : s.safe;
       st.ebase[k] = static_cast<int64_t>(ei) * P::DPA * a.C_k + (lane >> 5) * TM::VEC;
     });
   }
@@ -712,6 +711,7 @@ struct Gemm {
             w[i] = o * tg[i];
           }
           store16(g + static_cast<int64_t>(row) * a.C_n, w);
+          __builtin_amdgcn_sched_barrier(0);  // one row at a time (register pressure)
         });
 #pragma unroll
         for (int i = 0; i < 16; ++i) w[i] = dg[i] * (1.0f - tg[i] * tg[i]);
@@ -755,30 +755,40 @@ struct Gemm {
       constexpr int rt = decltype(RTI)::value;
       constexpr int sb = P::tab.base[lo] + rt * P::ntype(lo);
       const int ei = s.eid[rt * 32 + (lane & 31)];
-      const int64_t eis = ei >= 0 ? ei : s.eid[0];
+      const int64_t eis = ei >= 0 ? ei : s.safe;
       const typename TM::raw* rsave = reinterpret_cast<const typename TM::raw*>(a.rsave) +
                                       eis * P::DP * a.C_n + col;
-      static_for<1 + (lo < M ? lo : M)>([&](auto MI) {
-        constexpr int m = decltype(MI)::value;
+      // 16-byte pieces at a time: fp32 rows eight channels, bf16 rows all sixteen
+      constexpr int NC = sizeof(typename TM::raw) == 2 ? 16 : 8;
+      static_for<(1 + (lo < M ? lo : M)) * (16 / NC)>([&](auto MI) {
+        constexpr int m = decltype(MI)::value / (16 / NC), c0 = decltype(MI)::value % (16 / NC) * NC;
         constexpr int q0 = m == 0 ? 0 : 2 * m - 1, nqm = m == 0 ? 1 : 2;
-        const int64_t slot = rad_slot<L, M>(q0, lo, col, a.C_n);
-        float rv[16], dr[16];
-        load16(reinterpret_cast<const typename TM::raw*>(a.rad) + eis * rw + slot, rv);
+        const int64_t slot = rad_slot<L, M>(q0, lo, col, a.C_n) + c0;
+        const typename TM::raw* radp = reinterpret_cast<const typename TM::raw*>(a.rad) + eis * rw + slot;
+        float rv[NC], dr[NC];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) dr[i] = 0.f;
+        for (int k = 0; k < NC; k += 8) load_vec<TM, 8>(radp + k, *reinterpret_cast<float(*)[8]>(&rv[k]));
+#pragma unroll
+        for (int i = 0; i < NC; ++i) dr[i] = 0.f;
         static_for<nqm>([&](auto QI) {
           constexpr int q = q0 + decltype(QI)::value;
           constexpr int sl = sb + P::qtype(q, lo);
-          float rr[16];
-          load16(rsave + static_cast<int64_t>(P::mrow(q, lo)) * a.C_n, rr);
+          float rr[NC];
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            dr[i] = fmaf(acc[sl][i], rr[i], dr[i]);
-            acc[sl][i] *= rv[i];
+          for (int k = 0; k < NC; k += 8)
+            load_vec<TM, 8>(rsave + static_cast<int64_t>(P::mrow(q, lo)) * a.C_n + c0 + k,
+                            *reinterpret_cast<float(*)[8]>(&rr[k]));
+#pragma unroll
+          for (int i = 0; i < NC; ++i) {
+            dr[i] = fmaf(acc[sl][c0 + i], rr[i], dr[i]);
+            acc[sl][c0 + i] *= rv[i];
           }
         });
-        if (a.drad != nullptr && ei >= 0)
-          store16(reinterpret_cast<typename TM::raw*>(a.drad) + ei * rw + slot, dr);
+        if (a.drad != nullptr && ei >= 0) {
+          typename TM::raw* dp = reinterpret_cast<typename TM::raw*>(a.drad) + ei * rw + slot;
+#pragma unroll
+          for (int k = 0; k < NC; k += 8) store_vec<TM, 8>(dp + k, *reinterpret_cast<float(*)[8]>(&dr[k]));
+        }
         __builtin_amdgcn_sched_barrier(0);  // one block at a time (register pressure)
       });
     });
@@ -802,7 +812,7 @@ struct Gemm {
     const float4* Dp[RT];
     static_for<RT>([&](auto R) {
       constexpr int rt = decltype(R)::value;
-      const int e = s.eid[rt * 32 + co] >= 0 ? s.eid[rt * 32 + co] : s.eid[0];
+      const int ei = s.eid[rt * 32 + co], e = ei >= 0 ? ei : s.safe;
       Dp[rt] = reinterpret_cast<const float4*>(a.dk + static_cast<int64_t>(e) * P::WS + P::woff(lo));
     });
     float4 nxt[PB / 4];
@@ -874,6 +884,66 @@ struct Gemm {
     }
   }
 
+  // What follows the K loop: the tile's nvalid edges' outputs from the wave's
+  // accumulators.  buf: the wave's staging; st0..st2: where the gate values pass
+  // from their waves to the degrees' (P::GW).
+  template <int W, bool RAD>
+  static __device__ __forceinline__ void epilogue(f32x16 (&acc)[P::MSLOT], Smem& s, const Args& a, int cb, int lane,
+                                                  int nvalid, float* buf, char* st0, char* st1, char* st2) {
+    // segment ends of the tile: bit e set if edge e closes its segment
+    const int le = lane < TE ? lane : TE - 1, ln = le + 1 < TE ? le + 1 : le;
+    const uint64_t endmask = __ballot(lane < nvalid && (lane == nvalid - 1 || s.seg[ln] != s.seg[le]));
+    const int col = cb * CB + 16 * (lane >> 5);  // the lane's first channel
+    if constexpr (P::GW) {
+      // bias and pre-activation rows; the gate values through the stages (every
+      // wave passes both barriers); the activation; the stores
+      static_for<L + 1>([&](auto LO) {
+        constexpr int lo = decltype(LO)::value;
+        if constexpr (P::tab.owner[lo] == W) {
+          add_bias<lo>(acc, a, col);
+          if (a.gsave != nullptr) save_pre<lo>(acc, s, a, col, lane);
+        }
+      });
+      gate_rows<W>(acc, s, a, col, lane);
+      gate_out<W>(acc, st0, st1, st2, lane);
+      __syncthreads();
+      static_for<L + 1>([&](auto LO) {
+        constexpr int lo = decltype(LO)::value;
+        if constexpr (P::tab.owner[lo] == W) gate_act_gw<lo>(acc, st0, st1, st2, lane);
+      });
+      __syncthreads();  // gate values read before the stages are staging again
+      static_for<L + 1>([&](auto LO) {
+        constexpr int lo = decltype(LO)::value;
+        if constexpr (P::tab.owner[lo] == W) {
+          if constexpr (MODE == FWD_EDGE)
+            save_pre<lo, true>(acc, s, a, col, lane);
+          else
+            rotate_sum<W, lo>(acc, s, a, cb, buf, lane, endmask);
+        }
+      });
+      return;
+    }
+    static_for<L + 1>([&](auto LO) {
+      constexpr int lo = decltype(LO)::value;
+      if constexpr (P::tab.owner[lo] == W) {
+        if constexpr (!P::BWD) {
+          add_bias<lo>(acc, a, col);
+          if constexpr (GATE) {
+            if (a.gsave != nullptr) save_pre<lo>(acc, s, a, col, lane);
+            gate_act<lo>(acc);
+          }
+        } else if constexpr (RAD)
+          radial<lo>(acc, s, a, col, lane);
+        if constexpr (MODE == BWD_EDGE)
+          store_gate_bwd<lo>(acc, s, a, col, lane);
+        else if constexpr (MODE == FWD_EDGE)
+          save_pre<lo, true>(acc, s, a, col, lane);
+        else
+          rotate_sum<W, lo>(acc, s, a, cb, buf, lane, endmask);
+      }
+    });
+  }
+
   template <int W, int KR, bool RAD>
   static __device__ __forceinline__ void body(Smem& s, char* st0, char* st1, char* st2,
                                               const Args& a,
@@ -906,60 +976,37 @@ struct Gemm {
       foff += static_cast<int64_t>(nks) * P::nbfrag(LI);
     });
     __syncthreads();  // all A reads done before the stages become epilogue staging
+    epilogue<W, RAD>(acc, s, a, cb, lane, nvalid, wave_staging(wave, st0, st1, st2), st0, st1, st2);
+  }
 
-    // segment ends of the tile: bit e set if edge e closes its segment
-    const int le = lane < TE ? lane : TE - 1, ln = le + 1 < TE ? le + 1 : le;
-    const uint64_t endmask = __ballot(lane < nvalid && (lane == nvalid - 1 || s.seg[ln] != s.seg[le]));
-    const int col = cb * CB + 16 * (lane >> 5);  // the lane's first channel
-    if constexpr (P::GW) {
-      // bias and pre-activation rows; the gate values through the stages (every
-      // wave passes the three barriers); the activation; the stores
-      float* tb = wave_staging(wave, st0, st1, st2);
-      static_for<L + 1>([&](auto LO) {
-        constexpr int lo = decltype(LO)::value;
-        if constexpr (P::tab.owner[lo] == W) {
-          add_bias<lo>(acc, a, col);
-          if (a.gsave != nullptr) save_pre<lo>(acc, s, a, col, lane);
-        }
-      });
-      gate_rows<W>(acc, s, a, col, lane);
-      gate_out<W>(acc, st0, st1, st2, lane);
-      __syncthreads();
-      static_for<L + 1>([&](auto LO) {
-        constexpr int lo = decltype(LO)::value;
-        if constexpr (P::tab.owner[lo] == W) gate_act_gw<lo>(acc, st0, st1, st2, lane);
-      });
-      __syncthreads();  // gate values read before the stages are staging again
-      static_for<L + 1>([&](auto LO) {
-        constexpr int lo = decltype(LO)::value;
-        if constexpr (P::tab.owner[lo] == W) {
-          if constexpr (MODE == FWD_EDGE)
-            save_pre<lo, true>(acc, s, a, col, lane);
-          else
-            rotate_sum<W, lo>(acc, s, a, cb, tb, lane, endmask);
-        }
-      });
-      return;
-    }
-    static_for<L + 1>([&](auto LO) {
-      constexpr int lo = decltype(LO)::value;
-      if constexpr (P::tab.owner[lo] == W) {
-        if constexpr (!P::BWD) {
-          add_bias<lo>(acc, a, col);
-          if constexpr (GATE) {
-            if (a.gsave != nullptr) save_pre<lo>(acc, s, a, col, lane);
-            gate_act<lo>(acc);
-          }
-        } else if constexpr (RAD)
-          radial<lo>(acc, s, a, col, lane);
-        if constexpr (MODE == BWD_EDGE)
-          store_gate_bwd<lo>(acc, s, a, col, lane);
-        else if constexpr (MODE == FWD_EDGE)
-          save_pre<lo, true>(acc, s, a, col, lane);
+  // The tile's edges (e0 .. e0 + nvalid - 1, may be none) and where the segment
+  // that ends at each goes: by the tile's threads 0 .. TE - 1, before a barrier.
+  // Segments cut by the tile boundary go to the partials buffer: the tile's
+  // first segment (slot 0) if it began in an earlier tile, its last one (slot 1)
+  // if it continues into the next tile.
+  static __device__ __forceinline__ void setup(Smem& s, const Args& a, int64_t tile, int64_t e0, int nvalid, int tid,
+                                               int safe) {
+    if (tid < TE) {
+      int sg = -1, ei = -1;
+      float* dst = nullptr;
+      if (tid < nvalid) {
+        const int64_t p = e0 + tid, el = e0 + nvalid - 1;
+        const int s0 = a.seg[e0], s1 = a.seg[el];
+        const bool fp = e0 > 0 && a.seg[e0 - 1] == s0;
+        const bool lp = el + 1 < a.E && a.seg[el + 1] == s1;
+        sg = a.seg[p];
+        ei = a.eidx ? a.eidx[p] : static_cast<int>(p);
+        const int64_t ow = a.ow > 0 ? a.ow : a.C_n;
+        if ((sg == s0 && fp) || (sg == s1 && lp))
+          dst = a.part + (tile * 2 + (sg == s0 ? 0 : 1)) * d * ow;
         else
-          rotate_sum<W, lo>(acc, s, a, cb, wave_staging(wave, st0, st1, st2), lane, endmask);
+          dst = a.out + static_cast<int64_t>(sg) * d * ow;
       }
-    });
+      s.seg[tid] = sg;
+      s.eid[tid] = ei;
+      s.optr[tid] = dst;
+    }
+    if (tid == 0) s.safe = safe;
   }
 
   template <int KR, bool RAD>
@@ -980,31 +1027,8 @@ struct Gemm {
     if (tile >= a.ntiles) return;  // whole workgroup exits together
     const int64_t e0 = tile * TE;
     const int nvalid = static_cast<int>((a.E - e0) < TE ? (a.E - e0) : TE);
-    if (tid < TE) {
-      const bool v = tid < nvalid;
-      const int64_t p = e0 + tid;
-      s.seg[tid] = v ? a.seg[p] : -1;
-      s.eid[tid] = v ? (a.eidx ? a.eidx[p] : static_cast<int>(p)) : -1;
-    }
+    setup(s, a, tile, e0, nvalid, tid, a.eidx ? a.eidx[e0] : static_cast<int>(e0));
     __syncthreads();
-    // Segments cut by the tile boundary go to the partials buffer: the tile's
-    // first segment (slot 0) if it began in an earlier tile, its last one
-    // (slot 1) if it continues into the next tile.
-    const bool fp = (e0 > 0) && (a.seg[e0 - 1] == a.seg[e0]);
-    const bool lp = (e0 + nvalid < a.E) && (a.seg[e0 + nvalid] == a.seg[e0 + nvalid - 1]);
-    if (tid < TE) {
-      float* dst = nullptr;
-      const int64_t ow = a.ow > 0 ? a.ow : a.C_n;
-      if (tid < nvalid) {
-        const int sg = s.seg[tid];
-        const bool first = sg == s.seg[0], last = sg == s.seg[nvalid - 1];
-        if ((first && fp) || (last && lp))
-          dst = a.part + (tile * 2 + (first ? 0 : 1)) * d * ow;
-        else
-          dst = a.out + static_cast<int64_t>(sg) * d * ow;
-      }
-      s.optr[tid] = dst;
-    }
     static_for<NW>([&](auto WI) {
       constexpr int w = decltype(WI)::value;
       if (wave == w) body<w, KR, RAD>(s, st0, st1, st2, a, cb, tid, nvalid);

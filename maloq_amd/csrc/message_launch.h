@@ -1,6 +1,6 @@
 #pragma once
 // Host-side launch helpers shared by the per-lmax instantiation files.
-#include "message_gemm.h"
+#include "message_split.h"
 
 namespace maloq {
 namespace msg {
@@ -35,8 +35,22 @@ struct Cfg {
   static constexpr int MINB = (L > 4 || (FULL && GATE && (MODE == FWD || MODE == FWD_EDGE))) ? 1 : 2;
 };
 
-inline int tile_edges(int lmax, int mmax, int gate, int mode = FWD) {
+// fp32 (SplitGemm): row tiles of 32 edges per group of four waves.  256 registers
+// per wave (two groups on a CU) hold two row tiles at lmax <= 4 without gate rows
+// among the outputs, one otherwise; mmax = lmax = 6 holds one only with 512 (one
+// group).
+template <int L, int M, bool GATE, int MODE>
+struct SplitCfg {
+  static constexpr bool FULL = M == L && L > 2;
+  static constexpr int RT = (FULL || L > 4 || (GATE && MODE != BWD_DX)) ? 1 : 2;
+  static constexpr bool PAIR = !(FULL && L > 4);  // built with two groups per workgroup too
+  static constexpr bool HALVE = L <= 4;  // and with two on one tile (lmax 6: 172 KB of stages)
+};
+
+// Edges per tile (the unit of the partial-segment buffers) of a kernel shape.
+inline int tile_edges(int dtype, int lmax, int mmax, int gate, int mode = FWD) {
   if (mmax == lmax && lmax > 2) return 32;
+  if (dtype == 0) return (lmax > 4 || (gate && mode != BWD_DX)) ? 32 : 64;
   return (mode == BWD_DX || lmax > 4 || !gate) ? 64 : 32;
 }
 // Every instantiation's tile has a multiple of 32 edges: partial-segment
@@ -53,25 +67,55 @@ void launch_kr(const Args& a, dim3 g, dim3 b, hipStream_t s) {
     hipLaunchKernelGGL((gemm_kernel<L, M, GATE, C::NW, C::RT, TM, MODE, KR, false, C::MINB>), g, b, 0, s, a);
 }
 
+// XCD-aware grids: tile groups in eights (one per XCD), n_cb workgroups per group.
+inline int64_t gemm_grid(int64_t groups, int n_cb) { return (groups + 7) / 8 * 8 * n_cb; }
+
+template <int L, int M, bool GATE, int MODE, int NG, int KS>
+int launch_split(const Args& a, hipStream_t s) {
+  using C = SplitCfg<L, M, GATE, MODE>;
+  const int64_t grid = gemm_grid((a.ntiles + NG - 1) / NG, a.n_cb);
+  MALOQ_REQUIRE(grid < (int64_t(1) << 31), "grid too large");
+  const dim3 g(static_cast<unsigned>(grid)), b(256 * NG * KS);
+  if (MODE == BWD_DX && a.rad != nullptr)
+    hipLaunchKernelGGL((split_gemm_kernel<L, M, GATE, C::RT, NG, KS, MODE, MODE == BWD_DX>), g, b, 0, s, a);
+  else
+    hipLaunchKernelGGL((split_gemm_kernel<L, M, GATE, C::RT, NG, KS, MODE, false>), g, b, 0, s, a);
+  return check_launch("split_gemm_kernel");
+}
+
 template <int L, int M, bool GATE, class TM, class TX, int MODE>
 int launch(const Args& a, hipStream_t s) {
-  constexpr int NW = Cfg<L, M, GATE, MODE>::NW, RT = Cfg<L, M, GATE, MODE>::RT;
-  MALOQ_REQUIRE(tile_edges(L, M, GATE, MODE) == 32 * RT, "tile size mismatch");
-  using P = GPlan<L, M, GATE, NW, RT>;
-  // Must match the workgroup -> (tile, channel block) mapping of Gemm::run:
-  // tiles in groups of 8 (one per XCD), n_cb workgroups per tile.
-  const int64_t grid = ((a.ntiles + 7) / 8) * 8 * a.n_cb;
-  MALOQ_REQUIRE(grid < (int64_t(1) << 31), "grid too large");
-  const dim3 g(static_cast<unsigned>(grid)), b(P::NT);
-  // the A-stage ring position of each K step is static per nks % 3 (nks >= 2)
-  const int nks = a.C_k / TM::KC;
-  switch (nks >= 2 ? nks % 3 : 3) {
-    case 0: launch_kr<L, M, GATE, TM, MODE, 0>(a, g, b, s); break;
-    case 1: launch_kr<L, M, GATE, TM, MODE, 1>(a, g, b, s); break;
-    case 2: launch_kr<L, M, GATE, TM, MODE, 2>(a, g, b, s); break;
-    default: launch_kr<L, M, GATE, TM, MODE, 3>(a, g, b, s); break;
+  if constexpr (std::is_same<TM, F32>::value) {
+    using C = SplitCfg<L, M, GATE, MODE>;
+    MALOQ_REQUIRE(tile_edges(0, L, M, GATE, MODE) == 32 * C::RT, "tile size mismatch");
+    // offsets into a channel block's weights and an edge's rows are 32-bit
+    MALOQ_REQUIRE(a.frags_per_cb < (int64_t(1) << 22) && a.C_k < (1 << 24), "too many channels");
+    // Two tiles per workgroup share the weights (30 000 edges, lmax 4, mmax 2, 128
+    // channels, input gradient with its prep: 1168 us, one tile each 1224).  Where one
+    // round of single tiles fits the compute units, one tile per workgroup and, where
+    // that is built, its K steps halved between two groups (420 edges, mmax = lmax = 4:
+    // 197 and 98 us for the two convolutions, not halved 269 and 133).
+    if constexpr (C::PAIR)
+      if (a.ntiles * a.n_cb > device_cus()) return launch_split<L, M, GATE, MODE, 2, 1>(a, s);
+    return launch_split<L, M, GATE, MODE, 1, C::HALVE ? 2 : 1>(a, s);
+  } else {
+    constexpr int NW = Cfg<L, M, GATE, MODE>::NW, RT = Cfg<L, M, GATE, MODE>::RT;
+    MALOQ_REQUIRE(tile_edges(1, L, M, GATE, MODE) == 32 * RT, "tile size mismatch");
+    using P = GPlan<L, M, GATE, NW, RT>;
+    // Must match the workgroup -> (tile, channel block) mapping of Gemm::run
+    const int64_t grid = gemm_grid(a.ntiles, a.n_cb);
+    MALOQ_REQUIRE(grid < (int64_t(1) << 31), "grid too large");
+    const dim3 g(static_cast<unsigned>(grid)), b(P::NT);
+    // the A-stage ring position of each K step is static per nks % 3 (nks >= 2)
+    const int nks = a.C_k / TM::KC;
+    switch (nks >= 2 ? nks % 3 : 3) {
+      case 0: launch_kr<L, M, GATE, TM, MODE, 0>(a, g, b, s); break;
+      case 1: launch_kr<L, M, GATE, TM, MODE, 1>(a, g, b, s); break;
+      case 2: launch_kr<L, M, GATE, TM, MODE, 2>(a, g, b, s); break;
+      default: launch_kr<L, M, GATE, TM, MODE, 3>(a, g, b, s); break;
+    }
+    return check_launch("gemm_kernel");
   }
-  return check_launch("gemm_kernel");
 }
 
 // The GEMM instantiations of one (lmax, mmax, dtype, mode), gated and not:

@@ -12,6 +12,9 @@ import math
 import pytest
 import torch
 
+from oracle import message as omsg
+from oracle import rotation as orot
+
 pytestmark = pytest.mark.gpu
 
 
@@ -53,3 +56,57 @@ def test_weight_gradient(lmax, mmax, c_in, c_out, gate, splits, E, device):
         ref = torch.cat([zp.T @ xp + zm.T @ xm, zm.T @ xp - zp.T @ xm])
         assert _rel(dwm[m - 1].cpu(), ref) < _tol(2 * E)
         at += 2 * k
+
+
+# Edge counts around the tiles (32 and 64 edges) of one group of waves, and large
+# enough for two groups per workgroup (256 workgroups and more) with a last group
+# that is empty or cut.
+@pytest.mark.parametrize("lmax,mmax,gate,E", [
+    (2, 2, False, 1), (4, 2, False, 63), (4, 2, False, 65), (4, 2, True, 33), (4, 4, False, 31), (4, 4, True, 33),
+    (6, 2, True, 33), (6, 6, False, 33),
+    (4, 2, False, 8192 + 1), (4, 2, False, 8192 + 65), (4, 4, True, 4096 + 1), (6, 2, True, 4096 + 40),
+])
+def test_block_forward_and_gradients(lmax, mmax, gate, E, device):
+    from maloq_amd import message as M
+    from maloq_amd.wigner import extract_euler_angles
+    C = 128 if E > 4000 else 32
+    N = max(2, E // 20)
+    gen = torch.Generator().manual_seed(E + lmax + mmax)
+    ei = torch.stack([torch.randint(0, N, (E,), generator=gen), torch.randint(0, N, (E,), generator=gen)])
+    k0 = (lmax + 1) * C
+    n0 = k0 + (lmax * C if gate else 0)
+    w = [torch.randn(n0, k0, generator=gen) / math.sqrt(k0), torch.randn(n0, generator=gen) * 0.1]
+    for m in range(1, mmax + 1):
+        k = (lmax - m + 1) * C
+        w.append(torch.randn(2 * k, k, generator=gen) / math.sqrt(2 * k))
+    x = torch.randn(N, (lmax + 1) ** 2, C, generator=gen)
+    rad = torch.rand(E, M.rad_width(lmax, mmax, C), generator=gen) + 0.5
+    gout = torch.randn(N, (lmax + 1) ** 2, C, generator=gen)
+    eul = extract_euler_angles(torch.randn(E, 3, generator=gen).to(device), seed=E)
+    plan = M.MessagePlan(ei.to(device), N)
+    dev = [t.to(device).requires_grad_() for t in (x, rad, *w)]
+    out = M.message_block(dev[0], plan, plan.sort_edges(eul), plan.sort_edges(dev[1]), dev[2], dev[3], dev[4:], lmax,
+                          mmax, gate=gate)
+    grads = torch.autograd.grad(out, dev, gout.to(device))
+    ref_in = [t.double().requires_grad_() for t in (x, rad, *w)]
+    e64 = eul.cpu().double()
+    ref = omsg.message_block(ref_in[0], ei, (e64[:, 0], e64[:, 1], e64[:, 2]), orot.load_jd(), lmax, mmax,
+                             {"w0": ref_in[2], "b0": ref_in[3], "wm": ref_in[4:], "c_out": C}, rad=ref_in[1], gate=gate)
+    ref_grads = torch.autograd.grad(ref, ref_in, gout.double())
+    # sums of up to 2 (lmax + 1) C products per row; the rotations and their fp32
+    # angles add as much again, on the way in and on the way out
+    n = 2 * k0
+    assert _rel(out.cpu(), ref.detach()) < 4 * _tol(n)
+    for got, want, terms in zip(grads, ref_grads, (n, n, E, E, *[2 * E] * mmax)):
+        assert _rel(got.cpu(), want) < 4 * _tol(max(n, terms))
+
+
+# K loops whose last step is half (channels an odd number of 8s) or that the two
+# groups of one tile cannot halve evenly; few edges and many (two tiles a workgroup).
+@pytest.mark.parametrize("c_in", [8, 24, 40, 96, 104])
+@pytest.mark.parametrize("lmax,mmax,E", [(2, 2, 50), (4, 2, 70), (4, 4, 70), (6, 2, 70), (4, 4, 8200)])
+def test_block_input_channels(lmax, mmax, E, c_in, device):
+    from test_message_hip import _run
+    _, got, ref = _run(lmax, mmax, torch.float32, lmax == 4, True, N=max(8, E // 20), E=E, c_in=c_in, c_out=32,
+                       seed=c_in, device=device)
+    assert _rel(got, ref) < 4 * _tol(2 * (lmax + 1) * c_in)
