@@ -29,7 +29,9 @@
 // fragment's lanes are read through a permutation that makes them consecutive).
 // Everything that is per edge in the epilogue is then per lane: its kept Wigner
 // entries, its saved rows, radial scales and gate rows are 16-byte loads and
-// stores of the lane's own edge, with no transposition through LDS.
+// stores of the lane's own edge, with no transposition through LDS.  (With lane =
+// channel those went through LDS, edge by edge: 45 000 edges, lmax 6, 128 channels,
+// bf16, gated 1105 us forward and 1087 input gradient, so 1023 and 1038.)
 // Epilogue per owned degree l: [bias, gate | radial scale and its gradient],
 // then for each pair of output columns (j, j+1) and each 32-edge row tile:
 // v = sum_q D(q, j) acc_q in the lane, written to a per-wave LDS tile

@@ -1,6 +1,6 @@
 #pragma once
 // Host-side launch helpers shared by the per-lmax instantiation files.
-#include "message_split.h"
+#include "message_ring.h"
 
 namespace maloq {
 namespace msg {
@@ -83,6 +83,24 @@ int launch_split(const Args& a, hipStream_t s) {
   return check_launch("split_gemm_kernel");
 }
 
+// bf16 (RingGemm): where a tile's accumulators leave the direct kernel one workgroup
+// per compute unit, a single wave per SIMD, and the grid is more than one round: the
+// gated accumulating forwards of mmax = lmax = 4.  36 800 edges, 128 channels: first
+// convolution of a layer 1190 us direct, 870 so; two waves a SIMD do as well directly
+// (its second, ungated: 393 and 440; lmax 6, mmax 2, 45 000 edges, gated: forward 1023
+// and 988, input gradient 1038 and 1045).
+template <int L, int M, bool GATE, int MODE>
+constexpr bool RING = L == 4 && M == L && GATE && (MODE == FWD || MODE == FWD_EDGE);
+
+template <int L, int M, bool GATE, int MODE>
+int launch_ring(const Args& a, hipStream_t s) {
+  const int64_t grid = gemm_grid((a.ntiles + 1) / 2, a.n_cb);
+  MALOQ_REQUIRE(grid < (int64_t(1) << 31), "grid too large");
+  hipLaunchKernelGGL((ring_gemm_kernel<L, M, GATE, 1, 2, MODE, false>), dim3(static_cast<unsigned>(grid)), dim3(512), 0,
+                     s, a);
+  return check_launch("ring_gemm_kernel");
+}
+
 template <int L, int M, bool GATE, class TM, class TX, int MODE>
 int launch(const Args& a, hipStream_t s) {
   if constexpr (std::is_same<TM, F32>::value) {
@@ -106,6 +124,8 @@ int launch(const Args& a, hipStream_t s) {
     const int64_t grid = gemm_grid(a.ntiles, a.n_cb);
     MALOQ_REQUIRE(grid < (int64_t(1) << 31), "grid too large");
     const dim3 g(static_cast<unsigned>(grid)), b(P::NT);
+    if constexpr (RING<L, M, GATE, MODE>)
+      if (grid > device_cus()) return launch_ring<L, M, GATE, MODE>(a, s);
     // the A-stage ring position of each K step is static per nks % 3 (nks >= 2)
     const int nks = a.C_k / TM::KC;
     switch (nks >= 2 ? nks % 3 : 3) {
