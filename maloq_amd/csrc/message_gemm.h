@@ -183,17 +183,10 @@ struct GPlan {
 typedef unsigned int frag_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ frag_t neg_frag(frag_t v, BF16) { return v ^ 0x80008000u; }
-__device__ __forceinline__ frag_t neg_frag(frag_t v, F32) { return v ^ 0x80000000u; }
 // acc += (weight fragment w)^T (row fragment a): accumulator rows are output
 // channels, columns (lanes) edges.
 __device__ __forceinline__ void mfma(f32x16& acc, frag_t a, frag_t w, BF16) {
   acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16((bf16x8)w, (bf16x8)a, acc, 0, 0, 0);
-}
-__device__ __forceinline__ void mfma(f32x16& acc, frag_t a, frag_t w, F32) {
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(w.x), __uint_as_float(a.x), acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(w.y), __uint_as_float(a.y), acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(w.z), __uint_as_float(a.z), acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(w.w), __uint_as_float(a.w), acc, 0, 0, 0);
 }
 
 // Byte offset in a packed weight fragment (lane i: column i & 31) that lane

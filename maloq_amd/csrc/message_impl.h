@@ -40,12 +40,6 @@ __device__ __forceinline__ void mma(f32x16& acc, const char* a, const char* b, i
   const bf16x8 bv = *reinterpret_cast<const bf16x8*>(b + lane * 16);
   acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc, 0, 0, 0);
 }
-__device__ __forceinline__ void mma(f32x16& acc, const char* a, const char* b, int lane, F32) {
-  const f32x4 av = *reinterpret_cast<const f32x4*>(a + lane * 16);
-  const f32x4 bv = *reinterpret_cast<const f32x4*>(b + lane * 16);
-#pragma unroll
-  for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[j], bv[j], acc, 0, 0, 0);
-}
 
 // Byte offset of element (row, k) inside an A/B fragment.
 template <class T>
@@ -53,13 +47,6 @@ __device__ __forceinline__ int frag_off(int row, int k);
 template <>
 __device__ __forceinline__ int frag_off<BF16>(int row, int k) {
   return (((k >> 3) * 32 + row) * 8 + (k & 7)) * 2;
-}
-template <>
-__device__ __forceinline__ int frag_off<F32>(int row, int k) {
-  // channel k of an 8-wide K step: lane half k/4, slot k%4.  MFMA j of the
-  // four 32x32x2 steps pairs channels j and 4+j in A and B alike, so the K
-  // order is a permutation shared by both operands and the sum is exact.
-  return (((k >> 2) * 32 + row) * 4 + (k & 3)) * 4;
 }
 
 // ------------------------------------------------------- compile-time plan
