@@ -1,6 +1,6 @@
 #pragma once
 // The SO(2) GEMM of the fused message block in bf16: the plans, epilogues and
-// outputs of message_gemm.h.
+// outputs of message_gemm.h, bit for bit.
 //
 // What bounds it: at one wave per 32 x 32 product block every weight fragment
 // (1 KB) feeds one MFMA (32 cycles) per row tile, and the four SIMDs of a compute
@@ -224,11 +224,19 @@ struct RingGemm {
             const frag_t wi = frag(B + S::bpos(LI, m, 2 * (lo - m) + 1) * FRAG);
             const frag_t wn = neg_frag(wi, BF16{});
             // forward: y+ += Wr x+ - Wi x-, y- += Wi x+ + Wr x-; input gradient:
-            // dx+ += Wr dy+ + Wi dy-, dx- += -Wi dy+ + Wr dy-
-            mul<sp, st>(acc, xp, wr);
-            mul<sm, st>(acc, xm, wr);
-            mul<sp, st>(acc, xm, P::BWD ? wi : wn);
-            mul<sm, st>(acc, xp, P::BWD ? wn : wi);
+            // dx+ += Wr dy+ + Wi dy-, dx- += -Wi dy+ + Wr dy-.  Each sum in the
+            // order of Gemm::mma_m, for the same bits.
+            if constexpr (!P::BWD) {
+              mul<sm, st>(acc, xp, wi);
+              mul<sp, st>(acc, xp, wr);
+              mul<sm, st>(acc, xm, wr);
+              mul<sp, st>(acc, xm, wn);
+            } else {
+              mul<sp, st>(acc, xp, wr);
+              mul<sm, st>(acc, xm, wr);
+              mul<sp, st>(acc, xm, wi);
+              mul<sm, st>(acc, xp, wn);
+            }
           }
         });
       }
