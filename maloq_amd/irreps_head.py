@@ -266,9 +266,18 @@ class _ColumnMap:
         self.csign = torch.as_tensor(sign[order], device=device)
 
 
+def _require_float(*tensors):
+    """The kernels read fp32 through bare pointers (a layer's output has another type
+    where a bias of another type promoted it, or under autocast)."""
+    for t in tensors:
+        if t.dtype != torch.float32:
+            raise ValueError(f"the irreps head computes in float32, not {t.dtype}")
+
+
 class _Gather(torch.autograd.Function):
     @staticmethod
     def forward(ctx, z, cmap):
+        _require_float(z)
         z = z.contiguous()
         out = torch.empty(z.shape[0], cmap.t, device=z.device, dtype=torch.float32)
         _lib.call("maloq_gather_columns", z, z.shape[1], z.shape[0], cmap.src, cmap.sign, cmap.t, out, cmap.t,
@@ -320,6 +329,7 @@ class _RowLinear(torch.autograd.Function):
 class _GateFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, s, lmax, act):
+        _require_float(x, s)
         out = torch.empty_like(x)
         cst = _cst(act)
         _lib.call("maloq_irreps_gate_fwd", x, x.shape[0], lmax, x.shape[2], s, cst, act, out,
@@ -417,6 +427,17 @@ def _ints(v):
 
 def _pointers(ts):
     return (ctypes.c_void_p * len(ts))(*[None if t is None else t.data_ptr() for t in ts])
+
+
+def _plain(x, lins):
+    """Whether the layers' parameters are what the fused kernels read through bare
+    pointers: float32 on x's device and whole.  The torch layers refuse the others
+    (or, for a bias of one element, expand it)."""
+    params = [t for lin in lins for t in (lin.weight, lin.bias)]
+    return (_lib.eager(x, *params) and all(t.dtype == torch.float32 and t.device == x.device and t.is_contiguous()
+                                           for t in params)
+            and all(lin.weight.numel() == lin.mul_in * lin.mul_out and lin.bias.numel() in (0, lin.mul_out)
+                    for lin in lins))
 
 
 class E3Linear(nn.Module):
@@ -538,7 +559,8 @@ class Fock_Irreps_Head(nn.Module):
         x = x.contiguous()
         ls = self.lin_scalars_learnable[spin]
         mul = [lin.mul_out for lin in lin_layers]
-        if x.shape[0] == 0 or x.data_ptr() % 16 or ls.weight.data_ptr() % 16 or not _lib.eager(x) or \
+        lins = [ls, *(lin for lin in lin_layers if lin.mul_out)]
+        if x.shape[0] == 0 or x.data_ptr() % 16 or ls.weight.data_ptr() % 16 or not _plain(x, lins) or \
                 not _lib.load().maloq_irreps_head_supported(self.lmax, self.sphere_channels, _ints(mul)):
             return _Gather.apply(self._z(x, lin_layers, spin), cmap)
         b0 = lin_layers[0].bias if lin_layers[0].bias.numel() else None

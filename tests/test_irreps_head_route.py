@@ -1,0 +1,97 @@
+"""Which calls Fock_Irreps_Head sends to the fused kernels, with the library replaced by
+a recorder: they read the parameters through bare pointers, so only whole float32
+parameters on the embeddings' device may go there.  Everything else goes to the torch
+layers, which refuse a wrong dtype or device."""
+import types
+
+import pytest
+import torch
+
+from maloq_amd import _lib
+from maloq_amd import tensor_decomp as ptd
+from maloq_amd.irreps_head import Fock_Irreps_Head
+
+L, C = 4, 32
+
+
+@pytest.fixture
+def calls(monkeypatch):
+    names = []
+    monkeypatch.setattr(_lib, "call", lambda name, *args: names.append(name))
+    monkeypatch.setattr(_lib, "load", lambda: types.SimpleNamespace(maloq_irreps_head_supported=lambda *a: 1))
+    monkeypatch.setattr(_lib, "require_cuda", lambda *t: None)
+    monkeypatch.setattr(_lib, "stream_of", lambda device: 0)
+    return names
+
+
+def _head():
+    t = ptd.BasisTables({1: [0, 0, 1], 6: [0, 0, 0, 1, 1, 2], 8: [0, 0, 0, 1, 1, 2]})
+    return Fock_Irreps_Head("+".join(f"{C}x{l}e" for l in range(L + 1)), t.req_output_irreps, L, C, ls_list=t.ls_list)
+
+
+def _run(head):
+    x = torch.randn(3, (L + 1) ** 2, C)
+    return head({"node_embeddings": x, "edge_embeddings": x}, None)
+
+
+def test_float32_parameters_are_fused(calls):
+    _run(_head())
+    assert calls == ["maloq_irreps_head_fwd"] * 2
+
+
+def _cast(dtype):
+    return lambda head: head.to(dtype)
+
+
+def _one(name, make):
+    """Replace one parameter."""
+    def change(head):
+        mod, _, leaf = name.rpartition(".")
+        mod = head.get_submodule(mod)
+        setattr(mod, leaf, torch.nn.Parameter(make(getattr(mod, leaf).detach())))
+    return change
+
+
+@pytest.mark.parametrize("change", [
+    _cast(torch.bfloat16), _cast(torch.float64),
+    _one("lin_scalars_learnable.0.weight", torch.Tensor.bfloat16),
+    _one("lin_scalars_learnable.0.bias", torch.Tensor.double),
+    _one("lin_out_layers.0.2.weight", torch.Tensor.half),
+    _one("lin_out_layers.0.0.bias", torch.Tensor.double),
+])
+def test_other_dtypes_are_refused(calls, change):
+    head = _head()
+    change(head)
+    with pytest.raises((RuntimeError, ValueError)):  # torch's layer, or a promoted result
+        _run(head)
+    assert "maloq_irreps_head_fwd" not in calls
+
+
+@pytest.mark.parametrize("name", ["lin_scalars_learnable.0.weight", "lin_scalars_learnable.0.bias",
+                                  "lin_out_layers.0.3.weight", "lin_out_layers.0.0.bias"])
+def test_parameters_elsewhere_are_not_fused(calls, name):
+    head = _head()
+    _one(name, lambda t: t.to("meta"))(head)
+    try:
+        _run(head)
+    except (RuntimeError, NotImplementedError):
+        pass
+    assert "maloq_irreps_head_fwd" not in calls
+
+
+def test_a_one_element_bias_is_expanded_by_the_layers(calls):
+    head = _head()
+    _one("lin_out_layers.0.0.bias", lambda t: t[:1].clone())(head)
+    _run(head)
+    assert "maloq_irreps_head_fwd" not in calls
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+def test_subclassed_parameters_are_not_fused(calls):
+    head = _head()
+    _one("lin_out_layers.0.1.weight", lambda t: t.as_subclass(_Sub))(head)
+    _run(head)
+    assert "maloq_irreps_head_fwd" not in calls
