@@ -153,11 +153,14 @@ def stream_of(device) -> int:
 
 
 def eager(*tensors) -> bool:
-    """Plain tensors outside torch.compile, tracing modes, functorch transforms and
-    forward-mode AD: where a call may go to a kernel that only eager code can see."""
+    """Plain tensors with memory of their own, outside torch.compile, tracing modes,
+    functorch transforms and forward-mode AD: where a call may go to a kernel that only
+    eager code can see.  (The batched gradients of ``is_grads_batched`` are plain in all
+    but their memory.)"""
     return (not torch.compiler.is_compiling() and torch._C._len_torch_dispatch_stack() == 0
             and torch._C._functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0
-            and all(t is None or type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors))
+            and all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and torch._C._has_storage(t))
+                    for t in tensors))
 
 
 def require_cuda(*tensors):

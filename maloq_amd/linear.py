@@ -58,10 +58,12 @@ class _RowsLinear(torch.autograd.Function):
     def backward(ctx, g):
         x, w = ctx.saved_tensors
         need_x, need_w, need_b = ctx.needs_input_grad
-        twice = torch.is_grad_enabled()  # create_graph: a gradient that can be differentiated again
+        # torch's products for a gradient that can be differentiated again
+        # (create_graph) or that is batched
+        kernels = not torch.is_grad_enabled() and _lib.eager(g, x, w)
         gx = g @ w if need_x else None
-        gw = (g.t() @ x if twice else rows_weight_grad(g, x)) if need_w else None
-        gb = (g.sum(0) if twice else rows_sum(g)) if need_b else None
+        gw = (rows_weight_grad(g, x) if kernels else g.t() @ x) if need_w else None
+        gb = (rows_sum(g) if kernels else g.sum(0)) if need_b else None
         return gx, gw, gb
 
 
