@@ -20,18 +20,21 @@ from . import _lib
 MIN_ROWS = 8192
 
 
-def _row_strided(t: torch.Tensor) -> torch.Tensor:
-    """``t``, or a copy where the kernel cannot step through its rows."""
-    return t if t.stride(1) == 1 and t.shape[1] <= t.stride(0) < 1 << 24 else t.contiguous()
+def _row_strided(t: torch.Tensor):
+    """``t``, or a copy where the kernel cannot step through its rows, and the row
+    stride (of a single row, whose own may be anything: its length)."""
+    n = t.shape[1]
+    ld = t.stride(0) if t.shape[0] > 1 else n
+    return (t, ld) if t.stride(1) == 1 and n <= ld < 1 << 24 else (t.contiguous(), n)
 
 
 def rows_weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     """``dy^T x`` [n, k] of fp32 GPU matrices dy [rows, n] and x [rows, k]."""
-    dy, x = _row_strided(dy), _row_strided(x)
+    (dy, ld_dy), (x, ld_x) = _row_strided(dy), _row_strided(x)
     rows, n, k = dy.shape[0], dy.shape[1], x.shape[1]
     parts = torch.empty(_lib.load().maloq_rows_dw_partials_floats(rows, n, k), device=dy.device, dtype=torch.float32)
     dw = torch.empty(n, k, device=dy.device, dtype=torch.float32)
-    _lib.call("maloq_rows_dw", dy, dy.stride(0), n, x, x.stride(0), k, rows, parts, dw, _lib.stream_of(dy.device))
+    _lib.call("maloq_rows_dw", dy, ld_dy, n, x, ld_x, k, rows, parts, dw, _lib.stream_of(dy.device))
     return dw
 
 

@@ -1,8 +1,12 @@
 """Which gradients of maloq_amd.linear go to this package's kernels, with these replaced
-by recorders: plain ones do; batched and twice differentiable ones are torch's."""
+by recorders: plain ones do; batched and twice differentiable ones are torch's.  And the
+row strides that the weight gradient's kernel is given."""
+import types
+
 import pytest
 import torch
 
+from maloq_amd import _lib
 from maloq_amd import linear as lin
 
 
@@ -53,3 +57,26 @@ def test_gradients_of_gradients(layer):
     for a, b in zip(twice(y), twice(ref)):
         torch.testing.assert_close(a, b)
     assert calls == []
+
+
+@pytest.mark.parametrize("make,ld", [
+    (lambda n: torch.randn(5, n), "n"),
+    (lambda n: torch.randn(5, n + 3)[:, 2:2 + n], "n + 3"),
+    (lambda n: torch.randn(n, 5).t(), "n"),                # a copy
+    (lambda n: torch.randn(1, n).expand(5, n), "n"),       # a copy
+    (lambda n: torch.randn(n, 1).t(), "n"),                # one row, of stride 1
+    (lambda n: torch.randn(4, n)[::4], "n"),               # one row, of stride 4 n
+    (lambda n: torch.randn(0, n), "n"),
+])
+@pytest.mark.parametrize("n", [1, 7])
+def test_row_strides(monkeypatch, make, ld, n):
+    seen = []
+    monkeypatch.setattr(_lib, "call", lambda name, *args: seen.append(args))
+    monkeypatch.setattr(_lib, "load", lambda: types.SimpleNamespace(maloq_rows_dw_partials_floats=lambda *a: 4))
+    monkeypatch.setattr(_lib, "stream_of", lambda device: 0)
+    dy = make(n)
+    lin.rows_weight_grad(dy, torch.randn(dy.shape[0], 3))
+    (got, stride, cols, _, ld_x, k, rows, *_), = seen
+    assert (stride, cols, ld_x, k, rows) == (eval(ld), n, 3, 3, dy.shape[0])
+    flat = torch.as_strided(got, (rows, n), (stride, 1))  # as the kernel steps through it
+    assert torch.equal(flat, dy)
