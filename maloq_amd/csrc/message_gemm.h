@@ -183,10 +183,18 @@ struct GPlan {
 typedef unsigned int frag_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ frag_t neg_frag(frag_t v, BF16) { return v ^ 0x80008000u; }
+__device__ __forceinline__ frag_t neg_frag(frag_t v, F32) { return v ^ 0x80000000u; }
 // acc += (weight fragment w)^T (row fragment a): accumulator rows are output
 // channels, columns (lanes) edges.
 __device__ __forceinline__ void mfma(f32x16& acc, frag_t a, frag_t w, BF16) {
   acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16((bf16x8)w, (bf16x8)a, acc, 0, 0, 0);
+}
+// Lane half h holds channels 4 h .. 4 h + 3 of an 8-wide K step: instruction j pairs
+// channels j and 4 + j of both operands.
+__device__ __forceinline__ void mfma(f32x16& acc, frag_t a, frag_t w, F32) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(w[j]), __uint_as_float(a[j]), acc, 0, 0, 0);
 }
 
 // Byte offset in a packed weight fragment (lane i: column i & 31) that lane

@@ -35,16 +35,23 @@ struct Cfg {
   static constexpr int MINB = (L > 4 || (FULL && GATE && (MODE == FWD || MODE == FWD_EDGE))) ? 1 : 2;
 };
 
-// fp32 (SplitGemm): row tiles of 32 edges per group of four waves.  256 registers
-// per wave (two groups on a CU) hold two row tiles at lmax <= 4 without gate rows
-// among the outputs, one otherwise; mmax = lmax = 6 holds one only with 512 (one
-// group).
+// fp32: on the bf16 matrix cores (SplitGemm) but for mmax = lmax = 6, whose
+// accumulators (13 row types of degree 6, one more with the gate) leave SplitGemm one
+// group of four waves per CU, one per SIMD, and spill in the gated forwards.  There the
+// fp32 units (Gemm) are faster: 9200 edges, 128 channels, forward 1412 us (SplitGemm
+// 1843), gated to the edge frame 3092 (3690), input gradient 1507 (1972), gated 1601
+// (2278).
+template <int L, int M>
+constexpr bool SPLIT = !(M == L && L > 4);
+
+// SplitGemm: row tiles of 32 edges per group of four waves.  256 registers per wave
+// (two groups on a CU) hold two row tiles at lmax <= 4 without gate rows among the
+// outputs, one otherwise.
 template <int L, int M, bool GATE, int MODE>
 struct SplitCfg {
   static constexpr bool FULL = M == L && L > 2;
   static constexpr int RT = (FULL || L > 4 || (GATE && MODE != BWD_DX)) ? 1 : 2;
-  static constexpr bool PAIR = !(FULL && L > 4);  // built with two groups per workgroup too
-  static constexpr bool HALVE = L <= 4;  // and with two on one tile (lmax 6: 172 KB of stages)
+  static constexpr bool HALVE = L <= 4;  // with two groups on one tile (lmax 6: 172 KB of stages)
 };
 
 // Edges per tile (the unit of the partial-segment buffers) of a kernel shape.
@@ -103,7 +110,7 @@ int launch_ring(const Args& a, hipStream_t s) {
 
 template <int L, int M, bool GATE, class TM, class TX, int MODE>
 int launch(const Args& a, hipStream_t s) {
-  if constexpr (std::is_same<TM, F32>::value) {
+  if constexpr (std::is_same<TM, F32>::value && SPLIT<L, M>) {
     using C = SplitCfg<L, M, GATE, MODE>;
     MALOQ_REQUIRE(tile_edges(0, L, M, GATE, MODE) == 32 * C::RT, "tile size mismatch");
     // offsets into a channel block's weights and an edge's rows are 32-bit
@@ -113,12 +120,11 @@ int launch(const Args& a, hipStream_t s) {
     // round of single tiles fits the compute units, one tile per workgroup and, where
     // that is built, its K steps halved between two groups (420 edges, mmax = lmax = 4:
     // 197 and 98 us for the two convolutions, not halved 269 and 133).
-    if constexpr (C::PAIR)
-      if (a.ntiles * a.n_cb > device_cus()) return launch_split<L, M, GATE, MODE, 2, 1>(a, s);
+    if (a.ntiles * a.n_cb > device_cus()) return launch_split<L, M, GATE, MODE, 2, 1>(a, s);
     return launch_split<L, M, GATE, MODE, 1, C::HALVE ? 2 : 1>(a, s);
   } else {
     constexpr int NW = Cfg<L, M, GATE, MODE>::NW, RT = Cfg<L, M, GATE, MODE>::RT;
-    MALOQ_REQUIRE(tile_edges(1, L, M, GATE, MODE) == 32 * RT, "tile size mismatch");
+    MALOQ_REQUIRE(tile_edges(std::is_same<TM, F32>::value ? 0 : 1, L, M, GATE, MODE) == 32 * RT, "tile size mismatch");
     using P = GPlan<L, M, GATE, NW, RT>;
     // Must match the workgroup -> (tile, channel block) mapping of Gemm::run
     const int64_t grid = gemm_grid(a.ntiles, a.n_cb);
