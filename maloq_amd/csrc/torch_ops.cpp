@@ -30,12 +30,15 @@
 //   edge_m0_rows, edge_degree_embed[_],          EdgeDegreeEmbedding (embedding.py:17-141):
 //   edge_degree_embed_bwd(...)                   m = 0 rows, the embedding (node: in place or a
 //                                                copy of x; edge), the gradient wrt the radial rows
-// Private helpers (CPU): _jd_table(), _pack_index(...) expose the tables the
-// operators build, for tests.
+// Private helpers: _jd_table(), _pack_index(...) expose the tables the operators
+// build, for tests (CPU); _rows_linear, _rows_weight_grad and _rows_sum are linear
+// layers over many rows (linear.py).
 #include <ATen/ATen.h>
 #include <ATen/hip/HIPContextLight.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/library.h>
 
 #include <algorithm>
@@ -609,6 +612,87 @@ std::vector<at::Tensor> weight_grads(const at::Tensor& dz, const at::Tensor& y, 
   res.push_back(db0);
   for (auto& t : dwm) res.push_back(t);
   return res;
+}
+
+// ------------------------------------------- linear layers over many rows
+// A matrix [rows, n] as the kernel steps through it: t, or a copy, and the row stride
+// (of a single row, whose own may be anything: its length).
+std::pair<at::Tensor, int64_t> row_strided(const at::Tensor& t) {
+  const int64_t n = t.size(1), ld = t.size(0) > 1 ? t.stride(0) : n;
+  if (t.stride(1) == 1 && n <= ld && ld < (int64_t(1) << 24)) return {t, ld};
+  return {t.contiguous(), n};
+}
+
+void require_rows(const at::Tensor& t, const char* what) {
+  require_gpu(t, what);
+  TORCH_CHECK_VALUE(t.dim() == 2 && t.scalar_type() == at::kFloat, what, " must be a float32 matrix");
+}
+
+// dy^T x [n, k] of dy [rows, n] and x [rows, k].
+at::Tensor rows_weight_grad(const at::Tensor& dy_, const at::Tensor& x_) {
+  require_rows(dy_, "dy");
+  require_rows(x_, "x");
+  const int64_t rows = dy_.size(0), n = dy_.size(1), k = x_.size(1);
+  TORCH_CHECK_VALUE(x_.size(0) == rows && x_.device() == dy_.device(), "dy and x must have the same rows and device");
+  const c10::DeviceGuard guard(dy_.device());
+  const auto dy = row_strided(dy_), x = row_strided(x_);
+  const int64_t nparts = maloq_rows_dw_partials_floats(rows, static_cast<int>(n), static_cast<int>(k));
+  at::Tensor parts = at::empty({std::max<int64_t>(1, nparts)}, dy_.options());
+  at::Tensor dw = at::empty({n, k}, dy_.options());
+  check_rc(maloq_rows_dw(dy.first.data_ptr<float>(), dy.second, static_cast<int>(n), x.first.data_ptr<float>(),
+                         x.second, static_cast<int>(k), rows, parts.data_ptr<float>(), dw.data_ptr<float>(), stream_of(dy_)),
+           "maloq_rows_dw");
+  return dw;
+}
+
+// Column sums [n] of dy [rows, n].
+at::Tensor rows_sum(const at::Tensor& dy_) {
+  require_rows(dy_, "dy");
+  const int64_t rows = dy_.size(0), n = dy_.size(1);
+  if (n % 4) return dy_.sum(0);
+  const c10::DeviceGuard guard(dy_.device());
+  const at::Tensor dy = dy_.contiguous();
+  const int64_t nparts = maloq_message_colsum_partials_floats(1, static_cast<int>(n), rows);
+  at::Tensor parts = at::empty({std::max<int64_t>(1, nparts)}, dy.options());
+  at::Tensor out = at::empty({n}, dy.options());
+  check_rc(maloq_message_colsum(0, dy.data_ptr(), 1, 0, 1, static_cast<int>(n), rows, parts.data_ptr<float>(),
+                                out.data_ptr<float>(), stream_of(dy)),
+           "maloq_message_colsum");
+  return out;
+}
+
+// Whether a gradient may go to the kernels: a plain one on the GPU.  One that can be
+// differentiated again (create_graph), a batched one (is_grads_batched, vmap: no
+// memory of its own) and one that something traces are torch's products.
+bool kernel_grad(const at::Tensor& g) {
+  return !at::GradMode::is_enabled() && g.is_cuda() && g.has_storage() && g.scalar_type() == at::kFloat &&
+         !g.key_set().has(c10::DispatchKey::Python) && !c10::impl::TorchDispatchModeTLS::any_modes_set();
+}
+
+// y = x w^T + b with the weight and bias gradients from the kernels above.  In C++: a
+// Python autograd function took 33 us of the host more per layer and training step,
+// more than the kernels save at 9000 rows.
+struct RowsLinear : torch::autograd::Function<RowsLinear> {
+  static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& x, const at::Tensor& w,
+                            const c10::optional<at::Tensor>& b) {
+    ctx->save_for_backward({x, w});
+    ctx->saved_data["bias"] = b.has_value();
+    return at::linear(x, w, b);
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const at::Tensor &x = saved[0], &w = saved[1], &g = grads[0];
+    const bool kernels = kernel_grad(g) && x.is_cuda() && x.has_storage();
+    at::Tensor gx, gw, gb;
+    if (ctx->needs_input_grad(0)) gx = g.mm(w);
+    if (ctx->needs_input_grad(1)) gw = kernels ? rows_weight_grad(g, x) : g.t().mm(x);
+    if (ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(2)) gb = kernels ? rows_sum(g) : g.sum(0);
+    return {gx, gw, gb};
+  }
+};
+at::Tensor rows_linear(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& b) {
+  return RowsLinear::apply(x, w, b);
 }
 
 // Gradients of message_block_fwd from its saved rows: [grad_x fp32 [N, d, c_in],
@@ -1381,6 +1465,9 @@ TORCH_LIBRARY(maloq_hip, m) {
   m.def("_jd_table() -> Tensor", &jd_table);
   m.def("_pack_index(int dtype_code, int lmax, int mmax, bool gate, int c_in, int c_out, int mode) -> Tensor",
         &pack_index_cpu);
+  m.def("_rows_linear(Tensor x, Tensor w, Tensor? b) -> Tensor", &rows_linear);
+  m.def("_rows_weight_grad(Tensor dy, Tensor x) -> Tensor", &rows_weight_grad);
+  m.def("_rows_sum(Tensor dy) -> Tensor", &rows_sum);
 }
 
 TORCH_LIBRARY_IMPL(maloq_hip, CUDA, m) {

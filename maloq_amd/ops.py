@@ -52,6 +52,11 @@ def _load_extension():
 _load_extension()
 _ops = torch.ops.maloq_hip
 
+# ------------------------------------- linear layers over many rows (linear.py)
+rows_linear = _ops._rows_linear
+rows_weight_grad = _ops._rows_weight_grad
+rows_sum = _ops._rows_sum
+
 # ------------------------------------------------------------------ Wigner
 edge_euler = _ops.edge_euler
 wigner_from_euler = _ops.wigner_from_euler

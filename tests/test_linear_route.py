@@ -1,82 +1,74 @@
-"""Which gradients of maloq_amd.linear go to this package's kernels, with these replaced
-by recorders: plain ones do; batched and twice differentiable ones are torch's.  And the
-row strides that the weight gradient's kernel is given."""
-import types
-
+"""The linear layer of maloq_amd.linear beside torch's, for every kind of gradient that
+a caller may ask of it: plain, batched and twice differentiable ones; and the row
+strides that the weight gradient's kernel meets."""
 import pytest
 import torch
 
-from maloq_amd import _lib
-from maloq_amd import linear as lin
+from maloq_amd import ops
 
 
-@pytest.fixture
-def layer(monkeypatch):
-    calls = []
-
-    def weight_grad(dy, x):
-        calls.append("weight")
-        return dy.t() @ x
-
-    def total(dy):
-        calls.append("bias")
-        return dy.sum(0)
-
-    monkeypatch.setattr(lin, "rows_weight_grad", weight_grad)
-    monkeypatch.setattr(lin, "rows_sum", total)
+def _layers(device, rows, needs=(True, True, True), bias=True):
     gen = torch.Generator().manual_seed(0)
-    leaves = [torch.randn(*s, generator=gen).requires_grad_() for s in ((9, 5), (3, 5), (3,))]
-    return calls, leaves, lin._RowsLinear.apply(*leaves), torch.nn.functional.linear(*leaves)
+    leaves = [torch.randn(*s, generator=gen).to(device).requires_grad_(n)
+              for s, n in zip(((rows, 8), (4, 8), (4,)), needs)]
+    args = leaves if bias else [*leaves[:2], None]
+    wanted = [t for t in args if t is not None and t.requires_grad]
+    return wanted, ops.rows_linear(*args), torch.nn.functional.linear(*args)
 
 
-def test_plain_gradients_use_the_kernels(layer):
-    calls, leaves, y, ref = layer
-    g = torch.randn(y.shape)
-    for a, b in zip(torch.autograd.grad(y, leaves, g), torch.autograd.grad(ref, leaves, g)):
-        torch.testing.assert_close(a, b)
-    assert calls == ["weight", "bias"]
+def _close(got, want, rows):
+    # sums of `rows` products in fp32, in other orders
+    for a, b in zip(got, want):
+        torch.testing.assert_close(a, b, rtol=1e-5, atol=2.0 ** -22 * rows ** 0.5 * 8)
 
 
-def test_batched_gradients(layer):
-    calls, leaves, y, ref = layer
-    g = torch.randn(4, *y.shape)
-    got = torch.autograd.grad(y, leaves, g, is_grads_batched=True, retain_graph=True)
-    mapped = torch.func.vmap(lambda v: torch.autograd.grad(y, leaves, v, retain_graph=True))(g)
-    want = torch.autograd.grad(ref, leaves, g, is_grads_batched=True)
-    for a, b, c in zip(got, mapped, want):
-        torch.testing.assert_close(a, c)
-        torch.testing.assert_close(b, c)
-    assert calls == []
+DEVICES = ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)]
 
 
-def test_gradients_of_gradients(layer):
-    calls, leaves, y, ref = layer
-    g = torch.randn(y.shape)
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("needs", [(True, True, True), (False, True, True), (True, False, True), (True, True, False)])
+def test_plain_gradients(device, needs, bias):
+    wanted, y, ref = _layers(device, 300, needs, bias)
+    g = torch.randn_like(y)
+    assert torch.equal(y, ref)
+    _close(torch.autograd.grad(y, wanted, g), torch.autograd.grad(ref, wanted, g), 300)
+
+
+@pytest.mark.parametrize("device", DEVICES)
+def test_batched_gradients(device):
+    wanted, y, ref = _layers(device, 300)
+    g = torch.randn(3, *y.shape, device=device)
+    got = torch.autograd.grad(y, wanted, g, is_grads_batched=True, retain_graph=True)
+    mapped = torch.func.vmap(lambda v: torch.autograd.grad(y, wanted, v, retain_graph=True))(g)
+    want = torch.autograd.grad(ref, wanted, g, is_grads_batched=True)
+    _close(got, want, 300)
+    _close(mapped, want, 300)
+
+
+@pytest.mark.parametrize("device", DEVICES)
+def test_gradients_of_gradients(device):
+    wanted, y, ref = _layers(device, 300)
+    g = torch.randn_like(y)
     twice = lambda out: torch.autograd.grad(
-        sum(t.square().sum() for t in torch.autograd.grad(out, leaves[:2], g, create_graph=True)), leaves[:2])
-    for a, b in zip(twice(y), twice(ref)):
-        torch.testing.assert_close(a, b)
-    assert calls == []
+        sum((t * t.detach().sign()).sum() for t in torch.autograd.grad(out, wanted[:2], g, create_graph=True)),
+        wanted[:2])
+    _close(twice(y), twice(ref), 300)
 
 
-@pytest.mark.parametrize("make,ld", [
-    (lambda n: torch.randn(5, n), "n"),
-    (lambda n: torch.randn(5, n + 3)[:, 2:2 + n], "n + 3"),
-    (lambda n: torch.randn(n, 5).t(), "n"),                # a copy
-    (lambda n: torch.randn(1, n).expand(5, n), "n"),       # a copy
-    (lambda n: torch.randn(n, 1).t(), "n"),                # one row, of stride 1
-    (lambda n: torch.randn(4, n)[::4], "n"),               # one row, of stride 4 n
-    (lambda n: torch.randn(0, n), "n"),
+@pytest.mark.gpu
+@pytest.mark.parametrize("make", [
+    lambda n: torch.randn(5, n, device="cuda"),
+    lambda n: torch.randn(5, n + 3, device="cuda")[:, 2:2 + n],
+    lambda n: torch.randn(n, 5, device="cuda").t(),              # a copy
+    lambda n: torch.randn(1, n, device="cuda").expand(5, n),     # a copy
+    lambda n: torch.randn(n, 1, device="cuda").t(),              # one row, of stride 1
+    lambda n: torch.randn(4, n, device="cuda")[::4],             # one row, of stride 4 n
+    lambda n: torch.randn(0, n, device="cuda"),
 ])
 @pytest.mark.parametrize("n", [1, 7])
-def test_row_strides(monkeypatch, make, ld, n):
-    seen = []
-    monkeypatch.setattr(_lib, "call", lambda name, *args: seen.append(args))
-    monkeypatch.setattr(_lib, "load", lambda: types.SimpleNamespace(maloq_rows_dw_partials_floats=lambda *a: 4))
-    monkeypatch.setattr(_lib, "stream_of", lambda device: 0)
+def test_row_strides(make, n, device):
+    from maloq_amd.linear import rows_weight_grad
     dy = make(n)
-    lin.rows_weight_grad(dy, torch.randn(dy.shape[0], 3))
-    (got, stride, cols, _, ld_x, k, rows, *_), = seen
-    assert (stride, cols, ld_x, k, rows) == (eval(ld), n, 3, 3, dy.shape[0])
-    flat = torch.as_strided(got, (rows, n), (stride, 1))  # as the kernel steps through it
-    assert torch.equal(flat, dy)
+    x = torch.randn(dy.shape[0], 3, device=device)
+    torch.testing.assert_close(rows_weight_grad(dy, x).cpu(), (dy.cpu().double().t() @ x.cpu().double()).float())
