@@ -371,6 +371,16 @@ def _z_rows(x, ws, bs, b0, wls, lmax, act):
     return torch.cat(zs, dim=1)
 
 
+def _fused_labels(x, ws, bs, b0, cmap, lmax, act, wls, scalars=None):
+    """maloq_irreps_head_fwd; ``scalars`` [rows, (1 + lmax) C] are kept for a backward."""
+    rows, C = x.shape[0], x.shape[2]
+    mul = [0 if w is None else w.shape[1] for w in wls]
+    out = torch.empty(rows, cmap.t, device=x.device, dtype=torch.float32)
+    _lib.call("maloq_irreps_head_fwd", x, rows, lmax, C, ws, bs, _pointers(wls), _ints(mul), b0, C ** -0.5,
+              _cst(act), act, cmap.src, cmap.sign, cmap.t, scalars, out, _lib.stream_of(x.device))
+    return out
+
+
 class _HeadFn(torch.autograd.Function):
     """Scalar linear, gate, per-degree linears and label gather in one launch
     (maloq_irreps_head_fwd), and the gradients in one (maloq_irreps_head_bwd) and
@@ -381,12 +391,11 @@ class _HeadFn(torch.autograd.Function):
     def forward(ctx, x, ws, bs, b0, cmap, lmax, act, *wls):
         x, ws = x.contiguous(), ws.contiguous()
         wls = [None if w is None else w.contiguous() for w in wls]
-        rows, C = x.shape[0], x.shape[2]
         mul = [0 if w is None else w.shape[1] for w in wls]
-        s = torch.empty(rows, ws.shape[1], device=x.device, dtype=torch.float32) if any(ctx.needs_input_grad) else None
-        out = torch.empty(rows, cmap.t, device=x.device, dtype=torch.float32)
-        _lib.call("maloq_irreps_head_fwd", x, rows, lmax, C, ws, bs, _pointers(wls), _ints(mul), b0, C ** -0.5,
-                  _cst(act), act, cmap.src, cmap.sign, cmap.t, s, out, _lib.stream_of(x.device))
+        s = None
+        if any(ctx.needs_input_grad):
+            s = torch.empty(x.shape[0], ws.shape[1], device=x.device, dtype=torch.float32)
+        out = _fused_labels(x, ws, bs, b0, cmap, lmax, act, wls, s)
         ctx.cmap, ctx.lmax, ctx.act, ctx.mul = cmap, lmax, act, mul
         ctx.takes_grad = ctx.needs_input_grad[:4] + ctx.needs_input_grad[7:]
         if s is not None:
@@ -565,8 +574,10 @@ class Fock_Irreps_Head(nn.Module):
             return _Gather.apply(self._z(x, lin_layers, spin), cmap)
         b0 = lin_layers[0].bias if lin_layers[0].bias.numel() else None
         raw = lambda lin: lin.weight.view(lin.mul_in, lin.mul_out)  # the kernels divide by sqrt(C)
-        return _HeadFn.apply(x, raw(ls), ls.bias if ls.bias.numel() else None, b0, cmap, self.lmax, self._act,
-                             *[raw(lin) if lin.mul_out else None for lin in lin_layers])
+        args = (x, raw(ls), ls.bias if ls.bias.numel() else None, b0, cmap, self.lmax, self._act)
+        wls = [raw(lin) if lin.mul_out else None for lin in lin_layers]
+        # (inside the function needs_input_grad is set in evaluation too)
+        return _HeadFn.apply(*args, *wls) if torch.is_grad_enabled() else _fused_labels(*args, wls)
 
     def _process(self, x, lin_layers, spin, stream):
         return self._labels(x, lin_layers, spin, self._column_map(stream, x.device))

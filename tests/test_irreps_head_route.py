@@ -14,10 +14,16 @@ from maloq_amd.irreps_head import Fock_Irreps_Head
 L, C = 4, 32
 
 
+class Calls(list):
+    def record(self, name, *args):
+        self.append(name)
+        self.args = args
+
+
 @pytest.fixture
 def calls(monkeypatch):
-    names = []
-    monkeypatch.setattr(_lib, "call", lambda name, *args: names.append(name))
+    names = Calls()
+    monkeypatch.setattr(_lib, "call", names.record)
     monkeypatch.setattr(_lib, "load", lambda: types.SimpleNamespace(maloq_irreps_head_supported=lambda *a: 1))
     monkeypatch.setattr(_lib, "require_cuda", lambda *t: None)
     monkeypatch.setattr(_lib, "stream_of", lambda device: 0)
@@ -95,3 +101,17 @@ def test_subclassed_parameters_are_not_fused(calls):
     _one("lin_out_layers.0.1.weight", lambda t: t.as_subclass(_Sub))(head)
     _run(head)
     assert "maloq_irreps_head_fwd" not in calls
+
+
+@pytest.mark.parametrize("mode,kept", [(torch.enable_grad, True), (torch.no_grad, False),
+                                       (torch.inference_mode, False)])
+def test_scalars_are_kept_for_a_backward_only(calls, mode, kept):
+    head = _head()
+    with mode():
+        _run(head)
+    scalars, out = calls.args[-3:-1]
+    assert (scalars is not None) == kept and out.shape[0] == 3
+    for p in head.parameters():
+        p.requires_grad_(False)
+    _run(head)
+    assert calls.args[-3] is None
