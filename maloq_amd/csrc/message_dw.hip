@@ -218,6 +218,7 @@ __global__ __launch_bounds__(SplitDw::NT) void dw_split_kernel(DwArgs a) {
   using S = SplitDw;
   constexpr int T = S::T, KE = S::KE, TI = S::TI, TJ = S::TJ;
   __shared__ alignas(16) char smem[2 * S::STAGE];
+  __shared__ int not_all_finite;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   // (32-bit and through readfirstlane: the compiler divides on the vector unit,
   // and what follows from the quotients should stay in scalar registers)
@@ -254,6 +255,7 @@ __global__ __launch_bounds__(SplitDw::NT) void dw_split_kernel(DwArgs a) {
   const float* src = reinterpret_cast<const float*>(op ? a.y : a.dz) + (eb + 8 * eh) * estride + col0;
 
   float r[2][8];
+  int again = 0;  // the sums are formed again, for infinite operands (split_bf16.h)
   auto load = [&](int step) {
     const int64_t left = ee - (eb + static_cast<int64_t>(step) * KE + 8 * eh);  // edges
     const int64_t bytes = left <= 0 ? 0 : ((left - 1) * estride + width - col0) * 4;
@@ -275,16 +277,11 @@ __global__ __launch_bounds__(SplitDw::NT) void dw_split_kernel(DwArgs a) {
 #pragma unroll
       for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4*>(dst + buf * S::STAGE + i * FRAG + c * 16) = pl[i];
     }
+    if (__builtin_expect(again, 0))
+      for (int c = 0; c < 2; ++c) fix_inf(dst + buf * S::STAGE + c * 16, FRAG);
   };
 
   f32x16 acc[TI][TJ];
-#pragma unroll
-  for (int i = 0; i < TI; ++i)
-#pragma unroll
-    for (int j = 0; j < TJ; ++j)
-#pragma unroll
-      for (int k = 0; k < 16; ++k) acc[i][j][k] = 0.f;
-
   const int wm = wave / S::WN, wn = wave % S::WN;
   const char* fa = smem + wm * TI * 3 * FRAG + lane * 16;
   const char* fb = smem + S::OP + wn * TJ * 3 * FRAG + lane * 16;
@@ -302,27 +299,53 @@ __global__ __launch_bounds__(SplitDw::NT) void dw_split_kernel(DwArgs a) {
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[split_a(k)], b[j][split_b(k)], acc[i][j], 0, 0, 0);
     }
   };
-  if (nsteps > 0) {
-    load(0);
-    store(0);
-    if (nsteps > 1) load(1);
-  }
-  __syncthreads();
-  for (int s = 0; s < nsteps; ++s) {
-    const int buf = s & 1;
-    bf16x8 b[TJ][3];
-#pragma unroll
-    for (int j = 0; j < TJ; ++j)
-#pragma unroll
-      for (int k = 0; k < 3; ++k) b[j][k] = *reinterpret_cast<const bf16x8*>(fb + buf * S::STAGE + (j * 3 + k) * FRAG);
-    rows(buf, 0, TI / 2, b);
-    // the other buffer was last read before the barrier that began this step
-    if (s + 1 < nsteps) {
-      store(buf ^ 1);
-      if (s + 2 < nsteps) load(s + 2);
+  if (tid == 0) not_all_finite = 0;
+#pragma unroll 1
+  for (;;) {
+    if (nsteps > 0) {
+      load(0);
+      store(0);
+      if (nsteps > 1) load(1);
     }
-    rows(buf, TI / 2, TI, b);
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < TJ; ++j)
+#pragma unroll
+        for (int k = 0; k < 16; ++k) acc[i][j][k] = 0.f;
     __syncthreads();
+    for (int s = 0; s < nsteps; ++s) {
+      const int buf = s & 1;
+      bf16x8 b[TJ][3];
+#pragma unroll
+      for (int j = 0; j < TJ; ++j)
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          b[j][k] = *reinterpret_cast<const bf16x8*>(fb + buf * S::STAGE + (j * 3 + k) * FRAG);
+      rows(buf, 0, TI / 2, b);
+      // the other buffer was last read before the barrier that began this step
+      if (s + 1 < nsteps) {
+        store(buf ^ 1);
+        if (s + 2 < nsteps) load(s + 2);
+      }
+      rows(buf, TI / 2, TI, b);
+      __syncthreads();
+    }
+    if (again) break;
+    float f[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < TJ; ++j)
+#pragma unroll
+        for (int k = 0; k < 16; ++k) f[k & 3] = not_finite(f[k & 3], acc[i][j][k]);
+    f[0] = (f[0] + f[1]) + (f[2] + f[3]);
+    if (f[0] != f[0]) not_all_finite = 1;
+    __syncthreads();
+    // (every wave's; the asm keeps two copies of the loop from being made of it)
+    again = __builtin_amdgcn_readfirstlane(not_all_finite);
+    asm volatile("" : "+s"(again));
+    if (__builtin_expect(!again, 1)) break;
   }
   const int row = tn * T + wm * TI * 32 + 4 * (lane >> 5);
   float* out = a.part + static_cast<int64_t>(split) * a.goff[a.ngroups] + a.goff[g];

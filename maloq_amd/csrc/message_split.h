@@ -141,6 +141,7 @@ struct SplitGemm {
     int nk, nbf;             // of degree li
     int foff;                // packed fragments before degree li's
     bool more;               // a kind is left
+    int again;               // sums formed again, for infinite operands (split_bf16.h)
   };
   static __device__ __forceinline__ int entry(const Ctx& c, int i) {
     int v = __builtin_amdgcn_readlane(c.tab[0], i & 63);
@@ -191,6 +192,7 @@ struct SplitGemm {
     }
   }
   static __device__ __forceinline__ void store(const Flight& n, const Ctx& c, char* buf, int lane) {
+    char* at = buf + c.wave * SF + lane * 16;
 #pragma unroll
     for (int k = 0; k < NS; ++k) {
       if (n.what[k] < 0) continue;
@@ -203,8 +205,15 @@ struct SplitGemm {
       uint4 pl[3];
       split8(r, pl);
 #pragma unroll
-      for (int i = 0; i < 3; ++i)
-        *reinterpret_cast<uint4*>(buf + (c.wave + NWT * k) * SF + i * FRAG + lane * 16) = pl[i];
+      for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4*>(at + NWT * k * SF + i * FRAG) = pl[i];
+    }
+    if (__builtin_expect(n.again, 0)) {
+      int held = 0;
+#pragma unroll
+      for (int k = 0; k < NS; ++k) held |= (n.what[k] >= 0) << k;
+#pragma unroll 1
+      for (int k = 0; k < NS; ++k)
+        if (held >> k & 1) fix_inf(at + NWT * k * SF, FRAG);
     }
   }
   static __device__ __forceinline__ void degree(Flight& n, const Ctx& c, int li) {
@@ -357,23 +366,56 @@ struct SplitGemm {
     cur = STAGE - cur;
   }
 
+  // The first kind into the stage at 0, the second's loads issued.
+  static __device__ __forceinline__ void begin(Flight& n, const Ctx& c, char* stages, int lane) {
+    n.more = true;
+    n.ks = c.ks0;
+    n.t = n.foff = 0;
+    degree(n, c, 0);
+    Addr at;
+    locate(at, n, c);
+    load(n, at);
+    store(n, c, stages, lane);
+    advance(n, c);
+    locate(at, n, c);
+    if (n.more) load(n, at);
+    __syncthreads();
+  }
+
   template <int W, bool RAD>
-  static __device__ __forceinline__ void body(typename G::Smem& s, char* pool, const Args& a, const Ctx& c, Flight& n,
-                                              int cb, int grp, int lane, int nvalid) {
+  static __device__ __forceinline__ void body(typename G::Smem& s, int* again, char* pool, const Args& a, const Ctx& c,
+                                              Flight& n, int cb, int grp, int lane, int nvalid) {
     char* stages = pool + (KS > 1 ? grp * 2 * STAGE : 0);
     f32x16 acc[P::MSLOT];
+#pragma unroll 1
+    for (n.again = 0;;) {
+      begin(n, c, stages, lane);
 #pragma unroll
-    for (int k = 0; k < P::MSLOT; ++k)
+      for (int k = 0; k < P::MSLOT; ++k)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[k][i] = 0.f;
-    int cur = 0;
-    static_for<L + 1>([&](auto LIc) {
-      constexpr int LI = decltype(LIc)::value;
-      for (int ks = 0; ks < c.nks; ++ks)
-        static_for<nkinds(LI)>([&](auto T) {
-          phase<W, LI, kind_at(LI, decltype(T)::value)>(acc, c, n, stages, cur, KS > 1 ? 0 : grp, lane);
-        });
-    });
+        for (int i = 0; i < 16; ++i) acc[k][i] = 0.f;
+      int cur = 0;
+      static_for<L + 1>([&](auto LIc) {
+        constexpr int LI = decltype(LIc)::value;
+        for (int ks = 0; ks < c.nks; ++ks)
+          static_for<nkinds(LI)>([&](auto T) {
+            phase<W, LI, kind_at(LI, decltype(T)::value)>(acc, c, n, stages, cur, KS > 1 ? 0 : grp, lane);
+          });
+      });
+      if (n.again) break;
+      float t[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < P::MSLOT; ++k)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) t[i & 3] = not_finite(t[i & 3], acc[k][i]);
+      t[0] = (t[0] + t[1]) + (t[2] + t[3]);
+      if (t[0] != t[0]) *again = 1;
+      __syncthreads();
+      // (every wave's; the asm keeps two copies of the loop from being made of it)
+      n.again = __builtin_amdgcn_readfirstlane(*again);
+      asm volatile("" : "+s"(n.again));
+      if (__builtin_expect(!n.again, 1)) break;
+    }
     // every wave is past its last read of the stages: they are staging now
     if constexpr (KS > 1) {
       constexpr int CH = POOL / (4 * FRAG * 4);  // accumulators at a time
@@ -414,6 +456,7 @@ struct SplitGemm {
   static __device__ __forceinline__ void run(const Args& a) {
     __shared__ typename G::Smem s[NG * KS];
     __shared__ alignas(16) char pool[POOL];
+    __shared__ int again;  // a sum is not finite
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // XCD-aware mapping, as in Gemm::run, over groups of NG tiles
@@ -429,6 +472,7 @@ struct SplitGemm {
     const int64_t e0 = tile * TE;
     const int nvalid = e0 < a.E ? static_cast<int>((a.E - e0) < TE ? (a.E - e0) : TE) : 0;
     G::setup(s[grp], a, tile, e0, nvalid, tid - 256 * grp, safe);
+    if (tid == 0) again = 0;
     Ctx c;
     {
       const int rt = wave % NR;  // staging row tile
@@ -445,23 +489,12 @@ struct SplitGemm {
       for (int r = 0; r < TREGS; ++r) c.tab[r] = stages.v[c.wave][64 * r + lane];
     }
     Flight n{};
-    n.more = true;
-    n.ks = c.ks0;
-    degree(n, c, 0);
-    Addr at;
-    locate(at, n, c);
-    load(n, at);
-    store(n, c, pool + (KS > 1 ? grp * 2 * STAGE : 0), lane);
-    advance(n, c);
-    locate(at, n, c);
-    if (n.more) load(n, at);
-    __syncthreads();
     // waves w and w + 4 share a SIMD: the second group's run the schedule backwards,
     // so that a heavy wave shares its SIMD with a light one
     const int sw = (wave & 3) ^ (grp & 1 ? 3 : 0);
     static_for<4>([&](auto WI) {
       constexpr int w = decltype(WI)::value;
-      if (sw == w) body<w, RAD>(s[grp], pool, a, c, n, cb, grp, lane, nvalid);
+      if (sw == w) body<w, RAD>(s[grp], &again, pool, a, c, n, cb, grp, lane, nvalid);
     });
   }
 };

@@ -110,3 +110,63 @@ def test_block_input_channels(lmax, mmax, E, c_in, device):
     _, got, ref = _run(lmax, mmax, torch.float32, lmax == 4, True, N=max(8, E // 20), E=E, c_in=c_in, c_out=32,
                        seed=c_in, device=device)
     assert _rel(got, ref) < 4 * _tol(2 * (lmax + 1) * c_in)
+
+
+# An infinity in the node features, the output gradient or a weight: what it reaches is
+# infinite, with the sign that a large number in its place gives, and the rest is finite.
+# (A permutation graph: no sum meets two infinities.)
+@pytest.mark.parametrize("where", ["x", "w0", "gout"])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+@pytest.mark.parametrize("lmax,mmax,E,C", [(4, 2, 70, 32), (6, 2, 70, 32), (6, 6, 70, 32), (4, 4, 2100, 128)])
+def test_infinite_inputs(lmax, mmax, E, C, sign, where, device):
+    from maloq_amd import message as M
+    from maloq_amd.wigner import extract_euler_angles
+    gen = torch.Generator().manual_seed(E + lmax)
+    ei = torch.stack([torch.randperm(E, generator=gen), torch.arange(E)])
+    k0 = (lmax + 1) * C
+    ts = {"x": torch.randn(E, (lmax + 1) ** 2, C, generator=gen),
+          "rad": torch.rand(E, M.rad_width(lmax, mmax, C), generator=gen) + 0.5,
+          "w0": torch.randn(k0, k0, generator=gen) / math.sqrt(k0), "b0": torch.randn(k0, generator=gen) * 0.1}
+    for m in range(1, mmax + 1):
+        k = (lmax - m + 1) * C
+        ts[f"w{m}"] = torch.randn(2 * k, k, generator=gen) / math.sqrt(2 * k)
+    gout = torch.randn(E, (lmax + 1) ** 2, C, generator=gen)
+    at = (5, 3) if where == "w0" else (7, 0, 3)
+    eul = extract_euler_angles(torch.randn(E, 3, generator=gen).to(device), seed=E)
+    plan = M.MessagePlan(ei.to(device), E)
+
+    def leaves(value, cast):
+        mine = {k: v.clone() for k, v in {**ts, "gout": gout}.items()}
+        mine[where][at] = value
+        g = cast(mine.pop("gout"))
+        return [cast(t).requires_grad_() for t in mine.values()], g
+
+    def results(out, ins, g):
+        return out.detach(), *torch.autograd.grad(out, ins, g)
+
+    dev, g = leaves(sign * math.inf, lambda t: t.to(device))
+    got = results(M.message_block(dev[0], plan, plan.sort_edges(eul), plan.sort_edges(dev[1]), dev[2], dev[3], dev[4:],
+                                  lmax, mmax), dev, g)
+    ref_in, g = leaves(sign * 2.0 ** 100, torch.Tensor.double)
+    e64 = eul.cpu().double()
+    want = results(omsg.message_block(ref_in[0], ei, (e64[:, 0], e64[:, 1], e64[:, 2]), orot.load_jd(), lmax, mmax,
+                                      {"w0": ref_in[2], "b0": ref_in[3], "wm": ref_in[4:], "c_out": C}, rad=ref_in[1]),
+                   ref_in, g)
+    for a, b in zip(got, want):
+        a, large = a.cpu(), b.abs() > 2.0 ** 60
+        assert torch.equal(a.isinf(), large) and torch.equal(a[large].sign(), b[large].sign().float())
+        assert a[~large].isfinite().all()
+    assert got[0].isinf().any() or where == "gout"
+
+
+def test_infinite_rows_of_a_weight_gradient(device):
+    from maloq_amd.linear import rows_weight_grad
+    gen = torch.Generator().manual_seed(0)
+    dy, x = torch.randn(300, 40, generator=gen), torch.randn(300, 33, generator=gen)
+    dy[17, 3], x[201, 8], x[202, 9] = -math.inf, math.inf, math.nan
+    dy[44, 5], x[44, 6] = math.inf, -math.inf
+    dy[50, 0] = x[50, 0] = 1.1 * 2.0 ** 66  # finite; their product is not
+    got = rows_weight_grad(dy.to(device), x.to(device)).cpu()
+    want = (dy.double().T @ x.double()).float()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[got.isinf()], want[want.isinf()])
