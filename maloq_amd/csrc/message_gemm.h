@@ -686,40 +686,63 @@ struct Gemm {
       const int64_t base = static_cast<int64_t>(ei) * DG * a.C_n + col;
       typename TM::raw* g = reinterpret_cast<typename TM::raw*>(a.zout) + base;
       const typename TM::raw* zs = reinterpret_cast<const typename TM::raw*>(a.gsave) + base;
-      float z[16], w[16];
-      if constexpr (lo == 0) {
-        load16(zs + static_cast<int64_t>(P::mrow(0, 0)) * a.C_n, z);
+      // Eight channels at a time, the next row's loads under this one's products, each
+      // row's offset found where it is used: sixteen channels and kept offsets spilled
+      // 320 bytes per lane at mmax = lmax = 4 in bf16 (36 800 edges, 128 channels: 733 us).
+      constexpr int VEC = TM::VEC, NU = 8 / VEC;
+      auto at = [&](int row, int c0) {
+        int64_t o = static_cast<int64_t>(row) * a.C_n + c0;
+        asm volatile("" : "+s"(o));
+        return o;
+      };
+      auto fetch = [&](uint4 (&u)[NU], int64_t o) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const float sg = 1.0f / (1.0f + expf(-z[i]));
-          w[i] = acc[sb][i] * (sg * (1.0f + z[i] * (1.0f - sg)));
-        }
-        store16(g + static_cast<int64_t>(P::mrow(0, 0)) * a.C_n, w);
-      } else {
-        float tg[16], dg[16];
-        load16(zs + static_cast<int64_t>(P::DP + lo - 1) * a.C_n, tg);
+        for (int k = 0; k < NU; ++k) u[k] = reinterpret_cast<const uint4*>(zs + o)[k];
+      };
+      auto unpack = [&](const uint4 (&u)[NU], float (&v)[8]) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          tg[i] = tanhf(tg[i]);
-          dg[i] = 0.f;
-        }
-        static_for<P::ntype(lo)>([&](auto TI) {
-          constexpr int t = decltype(TI)::value;
-          constexpr int row = P::mrow(t, lo);
-          load16(zs + static_cast<int64_t>(row) * a.C_n, z);
+        for (int k = 0; k < NU; ++k) unpack_vec<TM, VEC>(u[k], *reinterpret_cast<float(*)[VEC]>(&v[k * VEC]));
+      };
+      static_for<2>([&](auto HI) {
+        constexpr int c0 = 8 * decltype(HI)::value;
+        float z[8], w[8];
+        uint4 u[NU];
+        fetch(u, at(P::mrow(0, lo), c0));
+        if constexpr (lo == 0) {
+          unpack(u, z);
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const float o = acc[sb + t][i];
-            dg[i] = fmaf(o, z[i], dg[i]);
-            w[i] = o * tg[i];
+          for (int i = 0; i < 8; ++i) {
+            const float sg = 1.0f / (1.0f + expf(-z[i]));
+            w[i] = acc[sb][c0 + i] * (sg * (1.0f + z[i] * (1.0f - sg)));
           }
-          store16(g + static_cast<int64_t>(row) * a.C_n, w);
-          __builtin_amdgcn_sched_barrier(0);  // one row at a time (register pressure)
-        });
+          store_vec<TM, 8>(g + at(P::mrow(0, 0), c0), w);
+        } else {
+          float tg[8], dg[8];
+          load_vec<TM, 8>(zs + at(P::DP + lo - 1, c0), tg);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) w[i] = dg[i] * (1.0f - tg[i] * tg[i]);
-        store16(g + static_cast<int64_t>(P::DP + lo - 1) * a.C_n, w);
-      }
+          for (int i = 0; i < 8; ++i) {
+            tg[i] = tanhf(tg[i]);
+            dg[i] = 0.f;
+          }
+          static_for<P::ntype(lo)>([&](auto TI) {
+            constexpr int t = decltype(TI)::value;
+            unpack(u, z);
+            if constexpr (t + 1 < P::ntype(lo)) fetch(u, at(P::mrow(t + 1, lo), c0));
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              const float o = acc[sb + t][c0 + i];
+              dg[i] = fmaf(o, z[i], dg[i]);
+              w[i] = o * tg[i];
+            }
+            store_vec<TM, 8>(g + at(P::mrow(t, lo), c0), w);
+            __builtin_amdgcn_sched_barrier(0);  // one row at a time (register pressure)
+          });
+#pragma unroll
+          for (int i = 0; i < 8; ++i) w[i] = dg[i] * (1.0f - tg[i] * tg[i]);
+          store_vec<TM, 8>(g + at(P::DP + lo - 1, c0), w);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
     });
   }
 
