@@ -2,8 +2,8 @@
 at the edges of the kernel's 256 x 256 tiles and of its row splits, against 64
 bits, and the layer itself against torch's.
 
-Tolerance: as for the other fp32 products on the bf16 matrix cores (2^-23 per
-product, and n products added in fp32, 16 at a time, six times over), four times
+Tolerance: as for the other fp32 products on the bf16 matrix cores (below 2^-23 of a
+product rms, and n products added in fp32, 16 at a time, six times over), four times
 over, relative 2-norm.
 """
 import math
