@@ -3,11 +3,13 @@
 // scalar linear's weights backward.  Reference: Fock_Irreps_Head.process
 // (helm/esen_osh.py:894-1052); the formulas are those of irreps_head.hip.
 //
-// What bounds it: HBM.  The embeddings (d C floats a row) are read once forward,
-// read and their gradient written once backward; gated copies, per-degree copies
-// and the outputs before the gather stay in registers and LDS.  fp32 MFMA
-// (16x16x4) does the products: 107 k per row at lmax 4, C 128, half the time of the
-// row's bytes.  Forward and backward of 20 000 rows at C 128, 56 copies, as layers
+// What bounds it: the fp32 MFMA (16x16x4; 107 k products per row at lmax 4, C 128) and
+// the exchange through LDS between them, in tiles of 32 rows whose weights each
+// workgroup reads again, with one workgroup of eight waves per compute unit.  HBM is
+// only the floor: the embeddings (d C floats a row) are read once forward, read and
+// their gradient written once backward (20 000 rows at C 128: 150 us at the rate of a
+// copy); gated copies, per-degree copies and the outputs before the gather stay in
+// registers and LDS.  Forward and backward of those 20 000 rows, 56 copies, as layers
 // (gate kernels, a library product and its copies per degree) 2011 us, so 690; 8 rows
 // (launches) 1161 and 271.
 //

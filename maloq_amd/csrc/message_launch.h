@@ -95,7 +95,8 @@ int launch_split(const Args& a, hipStream_t s) {
 // gated accumulating forwards of mmax = lmax = 4.  36 800 edges, 128 channels: first
 // convolution of a layer 1190 us direct, 870 so; two waves a SIMD do as well directly
 // (its second, ungated: 393 and 440; lmax 6, mmax 2, 45 000 edges, gated: forward 1023
-// and 988, input gradient 1038 and 1045).
+// and 988, input gradient 1038 and 1045).  mmax = lmax = 6 is as short of waves, but
+// two of its stages (81 KB each) do not fit the LDS.
 template <int L, int M, bool GATE, int MODE>
 constexpr bool RING = L == 4 && M == L && GATE && (MODE == FWD || MODE == FWD_EDGE);
 

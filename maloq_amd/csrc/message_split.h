@@ -4,11 +4,12 @@
 //
 // What bounds it: six bf16 MFMAs stand for one fp32 product block, so a K step
 // of 16 channels is long (4800 cycles per CU at lmax 4, mmax 2) and the loads
-// are easily hidden; what competes with the MFMAs is the LDS (80 % as busy) and
-// the splitting of the operands on the VALU.  30 000 edges, lmax 4, mmax 2, 128
-// channels: forward 1290 us on the fp32 matrix instructions, so 1040; input gradient
-// 1429 and 1217.  Both ask for as much reuse of a
-// split fragment as the registers allow:
+// are easily hidden; what competes with the MFMAs is the splitting of the operands on
+// the VALU and the LDS reads (no bank conflicts).  36 800 edges, lmax 4, mmax 2, 128
+// channels: forward 1296 us on the fp32 matrix instructions, so 962 (928 TFLOP/s of
+// bf16 products, where a large library product reaches 1157); input gradient 1432
+// and 1239 (682: its epilogue with radial rows spills 200 bytes per lane).  Both ask
+// for as much reuse of a split fragment as the registers allow:
 //   * A workgroup owns NG tiles of 32 RT edges and CB = 32 kernel-output
 //     channels.  Four waves per tile own whole output degrees (the schedule of
 //     GPlan); the NG groups share the weights.
@@ -25,6 +26,8 @@
 //   * Where the tiles leave compute units idle, two groups of waves (KS = 2) halve
 //     one tile's K steps between them, each with stages of its own, so that one
 //     computes while the other waits; the second's sums are added to the first's.
+//   * A tile with a sum that is not finite runs its K loop once more, for infinite
+//     operands (split_bf16.h).
 #include "message_gemm.h"
 #include "split_bf16.h"
 

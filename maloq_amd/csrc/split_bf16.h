@@ -16,7 +16,7 @@
 // Range: the planes are bf16, whose least number is 2^-133, so that a float below
 // 2^-109 loses its last bits.  A product beyond the floats is infinite; from 2^144 on
 // it may be NaN (its parts are infinite too, and the third plane's may have the other
-// sign).  Infinite operands: see split8.
+// sign).  Infinite operands: see fix_inf.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

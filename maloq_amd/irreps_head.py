@@ -11,14 +11,17 @@ The reference's output head (helm/esen_osh.py:522-1064) maps the backbone's
 and the l-sorted result is permuted to the labels' irreps order (and, with
 reduce_node, expanded from the node-reduced irreps by index and parity sign).
 
-Here the features stay in the backbone's l-major layout (no stacked copy):
-the scalar and per-l linears are plain GEMMs on the library (torch.matmul ->
-hipBLASLt); the gate is ``maloq_irreps_gate_fwd`` / ``_bwd``; and one
-``maloq_gather_columns`` does the per-l transpose to e3nn's channel-major
-layout, the output permutation and the node expansion together (its gradient
-is the fixed-order ``maloq_scatter_columns``).  Parameter names follow the
-reference (e3nn Linear's flat ``weight`` [mul_in * mul_out] and ``bias``), so
-state dicts load.
+Here the features stay in the backbone's l-major layout (no stacked copy).  With
+up to 32 copies of a degree, as in the molecular bases, one kernel does all of it
+for 32 rows at a time, the label gather included, and one its gradients
+(``maloq_irreps_head_fwd`` / ``_bwd``).  Larger bases, tracing, second derivatives
+and parameters that are not whole float32 tensors on the embeddings' device take the
+layers one by one: the scalar and per-l linears are torch products; the gate is
+``maloq_irreps_gate_fwd`` / ``_bwd``; and one ``maloq_gather_columns`` does the
+per-l transpose to e3nn's channel-major layout, the output permutation and the node
+expansion together (its gradient is the fixed-order ``maloq_scatter_columns``).
+Parameter names follow the reference (e3nn Linear's flat ``weight``
+[mul_in * mul_out] and ``bias``), so state dicts load.
 
 With reduce_edge (esen_osh.py:570-575, 894-944, 1090-1130) every edge pair
 (i -> j, j -> i) is processed once as alpha = x_ij + x_ji and beta = x_ij - x_ji
@@ -350,8 +353,8 @@ class _GateFn(torch.autograd.Function):
 
 def _z_rows(x, ws, bs, b0, wls, lmax, act):
     """s = x_0 ws + bs, gate, per-l linear into Z [rows, sum_l (2l+1) mul_l]
-    (m-major per degree): one launch per step, for the shapes the fused kernels
-    are not built for."""
+    (m-major per degree), each as a product or kernel of its own: for the calls that
+    the fused kernels do not take, and for second derivatives of those they do."""
     s = _RowLinear.apply(x[:, 0, :], ws, bs)
     g = _GateFn.apply(x, s.contiguous(), lmax, act)
     # one flat [rows (2l+1), C] x [C, mul_l] GEMM per degree: split (its
