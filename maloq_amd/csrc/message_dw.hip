@@ -199,7 +199,7 @@ __global__ __launch_bounds__(256) void dw_kernel(DwArgs a) {
 // What bounds it: the bf16 matrix cores (six products for one), at a rate close
 // to that of the library's large bf16 product on this card (1.16 PFLOP/s).  lmax
 // 4, mmax 2, 128 channels, 36 800 edges, 15 splits (two rounds of workgroups),
-// sums and biases included: 1350 us on the fp32 units -> 862.  One round (7 splits) takes
+// sums and biases included: 1350 us on the fp32 units -> 840.  One round (7 splits) takes
 // 1011: its longest workgroup has nothing beside it, and its sums are longer (error
 // 1.33e-6 against 9.0e-7; the fp32 units 1.22e-6 at their 8 splits).  128-wide tiles
 // (twice the LDS reads and splitting per product) were no faster anywhere, also on

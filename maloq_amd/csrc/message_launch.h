@@ -93,7 +93,7 @@ int launch_split(const Args& a, hipStream_t s) {
 // bf16 (RingGemm): where a tile's accumulators leave the direct kernel one workgroup
 // per compute unit, a single wave per SIMD, and the grid is more than one round: the
 // gated accumulating forwards of mmax = lmax = 4.  36 800 edges, 128 channels: first
-// convolution of a layer 1190 us direct, 870 so; two waves a SIMD do as well directly
+// convolution of a layer 1190 us direct, 843 so; two waves a SIMD do as well directly
 // (its second, ungated: 393 and 440; lmax 6, mmax 2, 45 000 edges, gated: forward 1023
 // and 988, input gradient 1038 and 1045).  mmax = lmax = 6 is as short of waves, but
 // two of its stages (81 KB each) do not fit the LDS.

@@ -6,7 +6,7 @@
 // (1 KB) feeds one MFMA (32 cycles) per row tile, and the four SIMDs of a compute
 // unit together draw their operands at the rate of the LDS.  36 800 edges, mmax = lmax
 // = 4, 128 channels, first convolution: with the weights read from L2 by each wave, one
-// wave per SIMD, 1190 us; so 860 (MFMA 18 % busy, L2 hits 89 %: what is left is the
+// wave per SIMD, 1190 us; so 843 (MFMA 18 % busy, L2 hits 89 %: what is left is the
 // latency of a phase, with one workgroup per compute unit).
 //   * A workgroup owns NG groups of RT row tiles and CB = 32 kernel-output
 //     channels.  Four waves per group own whole output degrees (the schedule of

@@ -6,9 +6,9 @@
 // of 16 channels is long (4800 cycles per CU at lmax 4, mmax 2) and the loads
 // are easily hidden; what competes with the MFMAs is the splitting of the operands on
 // the VALU and the LDS reads (no bank conflicts).  36 800 edges, lmax 4, mmax 2, 128
-// channels: forward 1296 us on the fp32 matrix instructions, so 962 (928 TFLOP/s of
+// channels: forward 1296 us on the fp32 matrix instructions, so 957 (942 TFLOP/s of
 // bf16 products, where a large library product reaches 1157); input gradient 1432
-// and 1239 (682: its epilogue with radial rows spills 200 bytes per lane).  Both ask
+// and 1209 (727: its epilogue with radial rows spills 200 bytes per lane).  Both ask
 // for as much reuse of a split fragment as the registers allow:
 //   * A workgroup owns NG tiles of 32 RT edges and CB = 32 kernel-output
 //     channels.  Four waves per tile own whole output degrees (the schedule of
