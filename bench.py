@@ -32,6 +32,7 @@ import time
 
 PEAK_BF16 = 2.5e15      # dense MFMA, MI355X
 PEAK_FP32 = 157.3e12
+PEAK_FP32_SPLIT = PEAK_BF16 / 6  # fp32 as six bf16 products: the message GEMMs but for mmax = lmax = 6
 PEAK_HBM = 8.0e12
 
 
@@ -705,6 +706,13 @@ def sparse_basis_leg(sw, reps=30):
                          "frac": bpb * nb / tf / PEAK_HBM, "bytes_per_block": bpb}}
 
 
+def message_gemm(dtype, lmax, mmax, gate):
+    """The SO(2) forward GEMM that a large graph runs on, and its matrix units' peak."""
+    if dtype == "bf16":
+        return ("ring_gemm_kernel" if gate and lmax == mmax == 4 else "gemm_kernel"), PEAK_BF16
+    return ("gemm_kernel", PEAK_FP32) if lmax == mmax == 6 else ("split_gemm_kernel", PEAK_FP32_SPLIT)
+
+
 def message_leg(cfg, dtype, steps, warmup, cpu=True):
     """fwd+bwd of the fused block on configuration ``cfg``: edges/s, the fused
     forward launch's MFMA roofline, and the CPU baseline."""
@@ -715,14 +723,14 @@ def message_leg(cfg, dtype, steps, warmup, cpu=True):
     t_launch = fused_forward_launch_time(w, reps=10)
     L, Mm, C, E = w["L"], w["M"], w["C"], w["E"]
     f_edge = fused_flops_per_edge(L, Mm, C, C) + (gated_flops_extra(L, C, C) if w["gate"] else 0)
-    peak = PEAK_BF16 if dtype == "bf16" else PEAK_FP32
+    kernel, peak = message_gemm(dtype, L, Mm, w["gate"])
     gname = MESSAGE_CONFIGS[cfg][0]
     res = {"metric": "edges/s (fused block fwd+bwd)", "value": E / t_step, "ms_per_step": t_step * 1e3,
            "fwd_edges_per_s": E / t_fwd, "dtype": dtype,
            "config": {"workload": f"{cfg} fused message block fwd+bwd{' (gated)' if w['gate'] else ''}",
                       "graph": gname, "edges": E, "nodes": w["N"], "lmax": L, "mmax": Mm, "channels": C,
                       "gate": w["gate"], "rbf_cutoff_A": w["cutoff"]},
-           "roofline": {"kernel": f"maloq_message_fwd: prep + gemm_kernel<{L},{Mm}> + fixup", "bound": "mfma",
+           "roofline": {"kernel": f"maloq_message_fwd: prep + {kernel}<{L},{Mm}> + fixup", "bound": "mfma",
                         "achieved": f_edge * E / t_launch / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s",
                         "frac": f_edge * E / t_launch / peak, "flops_per_edge": f_edge,
                         "launch_ms": t_launch * 1e3}}
@@ -811,24 +819,41 @@ COUNTER_PIECES = (("step_config2_fp32", "config 2, fp32, training step"),
                   ("step_config2_bf16", "config 2, bf16, training step"),
                   ("step_config4_bf16", "config 4 (lmax 6, gated), bf16, training step"),
                   ("step_config5_bf16", "config 5 (C 256), bf16, training step"),
-                  ("edgewise_step_bf16", "Edgewise two convolutions, config 2, bf16, fwd+bwd"))
+                  ("edgewise_step_bf16", "Edgewise two convolutions, config 2, bf16, fwd+bwd"),
+                  ("ref-backbone_fp32", "Edgewise x4 at lmax = mmax = 4, fp32, fwd+bwd"),
+                  ("ref-backbone_bf16", "Edgewise x4 at lmax = mmax = 4, bf16, fwd+bwd"),
+                  ("fock-head_fp32", "Fock_Irreps_Head, config 3 batch, fwd+bwd"))
 SIMDS = 1024  # 256 CUs x 4 SIMDs
 
 
 def _kernel_label(name):
     """Short label of a message-block kernel from its demangled name, or None."""
     import re
-    m = re.search(r"gemm_kernel<(\d+), (\d+), (true|false), (\d+), (\d+), maloq::msg::(\w+), (\d+), (\d+), "
-                  r"(true|false), (\d+)>", name)
+    modes = {"0": "FWD", "1": "BWD_DX", "2": "FWD_EDGE", "3": "BWD_EDGE"}
+
+    def label(L, M, gate, mode, rad, what):
+        return (f"gemm {modes[mode]} L{L} M{M}{' gated' if gate == 'true' else ''} {what}"
+                f"{', radial grad' if rad == 'true' else ''})")
+
+    m = re.search(r" gemm_kernel<(\d+), (\d+), (true|false), (\d+), (\d+), maloq::msg::(\w+), (\d+), (\d+), "
+                  r"(true|false), (\d+)>", name.replace("::gemm_kernel", " gemm_kernel"))
     if m:
         L, M, gate, nw, rt, tm, mode, kr, rad, minb = m.groups()
-        modes = {"0": "FWD", "1": "BWD_DX", "2": "FWD_EDGE", "3": "BWD_EDGE"}
-        return (f"gemm {modes[mode]} L{L} M{M}{' gated' if gate == 'true' else ''} {tm} "
-                f"({32 * int(rt)}-edge tiles, {nw} waves{', radial grad' if rad == 'true' else ''})")
-    for k in ("dw_tr_kernel", "dw_kernel", "dw_reduce_kernel", "prep_kernel", "radial_fwd", "radial_du",
-              "radial_chain", "radial_dwo"):
+        return label(L, M, gate, mode, rad, f"{tm} ({32 * int(rt)}-edge tiles, {nw} waves")
+    m = re.search(r"split_gemm_kernel<(\d+), (\d+), (true|false), (\d+), (\d+), (\d+), (\d+), (true|false)>", name)
+    if m:
+        L, M, gate, rt, ng, ks, mode, rad = m.groups()
+        return label(L, M, gate, mode, rad, f"F32 as six bf16 products ({32 * int(rt)}-edge tiles, "
+                                            f"{4 * int(ng) * int(ks)} waves on {ng}")
+    m = re.search(r"ring_gemm_kernel<(\d+), (\d+), (true|false), (\d+), (\d+), (\d+), (true|false)>", name)
+    if m:
+        L, M, gate, rt, ng, mode, rad = m.groups()
+        return label(L, M, gate, mode, rad, f"BF16 weights through LDS ({32 * int(rt)}-edge tiles, "
+                                            f"{4 * int(ng)} waves on {ng}")
+    for k in ("head_fwd_kernel", "head_bwd_kernel", "dw_split_kernel", "dw_tr_kernel", "dw_kernel", "dw_reduce_kernel",
+              "prep_kernel", "radial_fwd", "radial_du", "radial_chain", "radial_dwo"):
         if k in name:
-            return k + ("<BF16>" if "BF16" in name and k == "dw_kernel" else "<F32>" if k == "dw_kernel" else "")
+            return k
     return None
 
 
@@ -839,12 +864,12 @@ def counters_from(root):
     SQ_INSTS_VALU_MFMA_MOPS_BF16 / _F32, SQ_INSTS_LDS, SQ_LDS_BANK_CONFLICT,
     SQ_LDS_IDX_ACTIVE).  Per kernel the median dispatch: MFMA busy = busy
     cycles over (SIMDs x the dispatch's cycles, from GRBM_GUI_ACTIVE per XCD
-    and its duration), MFMA TFLOP/s executed (MOPS x 512 over the duration),
-    LDS bank-conflict cycles per LDS-active cycle."""
+    and its duration), MFMA TFLOP/s executed (MOPS x 512 over the duration), LDS
+    active = LDS-active cycles over (CUs x the dispatch's cycles), LDS bank-conflict cycles per LDS-active cycle."""
     import csv
     import statistics
     rows = ["| workload | kernel | dispatch µs | MFMA busy | MFMA TFLOP/s executed | MFMA instr. | LDS instr. | "
-            "LDS bank conflicts / LDS active cycles |", "|---|---|---|---|---|---|---|---|"]
+            "LDS active | LDS bank conflicts / LDS active cycles |", "|---|---|---|---|---|---|---|---|---|"]
     for piece, what in COUNTER_PIECES:
         path = os.path.join(root, piece, "run_counter_collection.csv")
         if not os.path.exists(path):
@@ -871,23 +896,24 @@ def counters_from(root):
             busy = med("SQ_VALU_MFMA_BUSY_CYCLES") / (SIMDS * cycles) if cycles else 0.0
             mops = med("SQ_INSTS_VALU_MFMA_MOPS_BF16") + med("SQ_INSTS_VALU_MFMA_MOPS_F32")
             tflops = mops * 512 / (dur * 1e-9) / 1e12 if dur else 0.0
+            lds = med("SQ_LDS_IDX_ACTIVE") / (SIMDS // 4 * cycles) if cycles else 0.0
             conf = med("SQ_LDS_BANK_CONFLICT") / max(med("SQ_LDS_IDX_ACTIVE"), 1.0)
             rows.append(f"| {what} | {label} | {dur / 1e3:.1f} | {100 * busy:.1f} % | {tflops:.1f} | "
-                        f"{med('SQ_INSTS_MFMA'):.3g} | {med('SQ_INSTS_LDS'):.3g} | {conf:.3f} |")
+                        f"{med('SQ_INSTS_MFMA'):.3g} | {med('SQ_INSTS_LDS'):.3g} | {100 * lds:.1f} % | {conf:.3f} |")
     out = os.path.join(os.path.dirname(TRAFFIC_JSON), "gemm_counters.md")
     with open(out, "w") as f:
         f.write("# MFMA and LDS counters of the message-block kernels (rocprofv3 --pmc, median dispatch)\n\n")
-        f.write("Commands (GPU box, repo root, one counter pass per workload):\n\n")
+        f.write("Commands (MI355X, repo root, one counter pass per workload):\n\n")
         for piece, what in COUNTER_PIECES:
-            only = "edgewise-step" if piece.startswith("edgewise") else "step"
-            dt = piece.rsplit("_", 1)[1]
+            only, dt = piece.rsplit("_", 1)
+            only = "edgewise-step" if only.startswith("edgewise") else "step" if only.startswith("step") else only
             cfg = "" if only != "step" else f" --cfg {piece.split('_')[1]}"
             f.write(f"    timeout -s KILL 90 rocprofv3 --pmc {' '.join(PMC_GEMM)} --output-format csv "
                     f"-d <root>/{piece} -o run -- python bench.py --only {only} --dtype {dt}{cfg} --reps 2\n")
         f.write(f"    python bench.py --counters-from <root>\n\n")
         f.write("MFMA busy: SQ_VALU_MFMA_BUSY_CYCLES / (1024 SIMDs x the dispatch's cycles); the cycles are "
                 "GRBM_GUI_ACTIVE per XCD (the counter is summed over the XCDs).  MFMA TFLOP/s executed: "
-                "(SQ_INSTS_VALU_MFMA_MOPS_BF16 + _F32) x 512 / dispatch time (peaks: bf16 2500, fp32 157.3).  "
+                "(SQ_INSTS_VALU_MFMA_MOPS_BF16 + _F32) x 512 / dispatch time (peaks: bf16 2500, fp32 157.3; six bf16 products a term of an fp32 one).  "
                 "Durations are those of the counter run (kernels serialised).\n\n")
         f.write("\n".join(rows) + "\n")
     print(open(out).read())
@@ -1087,7 +1113,7 @@ def reference_backbone_leg(dtype_name, steps=5, warmup=2, cpu=True, lmax=4, laye
     t_fwd_nc = time_steps(lambda: reference_backbone_pass(rw, False, cached=False), steps, warmup)
     E, n = rw["E"], len(rw["mods"])
     fl = edgewise_flops_per_edge(rw["L"], rw["M"], rw["C"], rw["H"]) * E * n
-    peak = PEAK_BF16 if dtype_name == "bf16" else PEAK_FP32
+    peak = message_gemm(dtype_name, rw["L"], rw["M"], True)[1]
     out = {"metric": "edges/s per layer", "fwd_bwd": E * n / t_step, "fwd": E * n / t_fwd,
            "fwd_without_plan_cache": E * n / t_fwd_nc, "ms_per_pass_fwd_bwd": t_step * 1e3,
            "ms_per_pass_fwd": t_fwd * 1e3, "ms_per_pass_fwd_without_plan_cache": t_fwd_nc * 1e3,
@@ -1329,7 +1355,7 @@ def main(argv=None):
     print(f"[bench] fwd+bwd {t_step * 1e3:.3f} ms/step, {E / t_step:.4g} edges/s", file=sys.stderr, flush=True)
     t_fwd_launch = fused_forward_launch_time(w)
     f_edge = fused_flops_per_edge(w["L"], w["M"], w["C"], w["C"])
-    peak = PEAK_BF16 if args.dtype == "bf16" else PEAK_FP32
+    kernel, peak = message_gemm(args.dtype, w["L"], w["M"], w["gate"])
     achieved = f_edge * E / t_fwd_launch
     t_fwd_step = time_steps(lambda: message_step(w, False), args.steps, args.warmup)
     result = {
@@ -1349,7 +1375,7 @@ def main(argv=None):
                                "rotate->SO(2)->inverse rotate->segment sum, input/radial/weight grads",
                    "molecules": 32, "atoms_per_molecule": 40, "edges": E, "nodes": w["N"],
                    "lmax": w["L"], "mmax": w["M"], "channels": w["C"], "rbf": 8, "cutoff_A": 6.0},
-        "roofline": {"kernel": "maloq_message_forward: prep + gemm_kernel<4,2> + fixup", "bound": "mfma",
+        "roofline": {"kernel": f"maloq_message_forward: prep + {kernel}<{w['L']},{w['M']}> + fixup", "bound": "mfma",
                      "achieved": achieved / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s",
                      "frac": achieved / peak, "traffic": load_traffic(f"message_fwd_{args.dtype}"),
                      "flops_per_edge": f_edge, "launch_ms": t_fwd_launch * 1e3},
